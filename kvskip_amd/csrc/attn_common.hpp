@@ -21,17 +21,25 @@
 // dispatch gap of the merge kernel.
 //
 // Pipeline per wavefront: K(j) and V(j) are in flight when block j starts; after QK(j) the K
-// loads of block j+1 are issued, after PV(j) its V loads. The last block is peeled off the
-// loop so every load in the loop is unconditional (exact wait counts).
+// loads of block j+1 are issued, after PV(j) its V loads. Every load in the loop is unconditional
+// (exact wait counts): the MFMA engine's last block requests one past the head's range (zeros, no
+// memory access), the VALU engine peels its last block off.
 //
-// QK runs on one of two engines (chosen per launch, KVSKIP_AMD_QK=valu|mfma):
-//   mfma  v_mfma_f32_16x16x32_bf16 with the G query heads as the 16 M rows (zero-padded), 16
-//         tokens as N and 32 dims as K: Q is 4 VGPRs per 32 dims whatever G, a 64-token block
-//         is 4 x (D/32) MFMAs, and the scores come out as lane (j = lane/16, c = lane%16)
-//         holding heads 4j..4j+3 of token c of each 16-token tile; block max / sum are 4-step
-//         DPP reductions inside the 16-lane row.
-//   valu  (below) dot products on v_dot2_f32_bf16.
-// Lane layouts (64 lanes, D = 64 or 128):
+// Two engines (chosen per launch, KVSKIP_AMD_QK=valu|mfma):
+//   mfma  both products on v_mfma_f32_16x16x32_bf16, nothing through LDS between them. Scores come out
+//         transposed: A = 16 tokens of K, B = the query heads as 16 columns, so a lane holds 16 scores
+//         of ONE head (column c = lane % 16) of a 64-token block, its softmax is in-lane arithmetic plus
+//         two lane swaps, and its weights already lie as the A operand of P V (row = lane % 16, tokens by
+//         lane / 16). V is read with 8 (D 64: 4) dims of a row per lane; two rows' halves are paired by
+//         v_perm into B operands whose column c is dim 8 c + j. Weights stay fp32: a weight is the exact
+//         sum of three bf16 parts (hi, mid, lo: 8 + 8 + 8 bits), and since the group's G <= 8 heads leave
+//         rows free, the 16 rows are the parts of the heads (4 heads x 3 parts, or 8 heads x hi, mid and
+//         a second product for lo): three parts for the price of one product. The products are exact and
+//         summed in fp32, as the VALU engine's.
+//         What it replaced: P through LDS and G x 128 FMAs plus 128 conversions per lane and block
+//         (D 128), which at G 7 took longer than the block's loads (figures at PFrag below).
+//   valu  (below) dot products on v_dot2_f32_bf16, P V on fp32 FMAs.
+// Lane layouts of the VALU engine (64 lanes, D = 64 or 128):
 //   K   8 lanes per token row, 8 rows per load; lane (r8 = lane/8, sub = lane%8) holds rows
 //       8*rg + r8 (rg = 0..7), dims [8 sub, 8 sub + 8) (+64 for D = 128), as packed bf16.
 //       QK = v_dot2_f32_bf16 against the unscaled bf16 query (exact products, fp32 sums),
@@ -425,46 +433,54 @@ __device__ __forceinline__ void reduce_acc_rows(float (&acc)[G][8]) {
     }
 }
 
-// LDS of the workgroup epilogue.
-template <int D, int G>
+// LDS of the workgroup epilogue. NP: parts of each accumulator (the MFMA engine's, PFrag::NP; 1 on the
+// VALU engine; 0: no accumulators, K only).
+template <int D, int G, int NP>
 struct MergeLds {
-  float acc[NWAVE * G * D];            // per-wavefront accumulators
-  float ml[NWAVE * G * 2];             // per-wavefront (m, l)
+  float acc[NP > 0 ? NWAVE * NP * G * D : 4];  // per-wavefront accumulators [wave][part][g][d]
+  float ml[NWAVE * G * 2];                     // per-wavefront (m, l)
 };
 
-// Workgroup epilogue: merge the wavefront states (m, l in log2 units, acc un-normalised), then
-// write out/out_f32/lse (one split) or the split partials.
-template <int D, int G, bool LOAD_V>
-__device__ __forceinline__ void finish(const AttnP& p, float (&m)[G], float (&l)[G], float (&acc)[G][8], int b,
-                                       int h, int split, MergeLds<D, G>& L, bool plain) {
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
-  constexpr int VLPR = Lay<D>::VLPR;
-  if constexpr (LOAD_V) {
-    reduce_acc_rows<D, G>(acc);
-    if (lane < VLPR) {
+// Accumulators of (head g, dim d) of every wavefront from the epilogue's LDS: the parts' sum, or the
+// first part where that is infinite (0 parts of a weight times an infinite V entry are NaN, and no part
+// of it). All reads are issued before any is used (the empty asm keeps the compiler from placing the
+// other parts' behind a branch on the first).
+template <int D, int G, int NP>
+__device__ __forceinline__ void merged_acc(float (&x)[NWAVE], const MergeLds<D, G, NP>& L, int g, int d) {
+  float part[NP][NWAVE];
 #pragma unroll
-      for (int g = 0; g < G; ++g)
+  for (int w = 0; w < NWAVE; ++w)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) L.acc[(wave * G + g) * D + 8 * lane + e] = acc[g][e];
+    for (int n = 0; n < NP; ++n) part[n][w] = L.acc[((w * NP + n) * G + g) * D + d];
+#pragma unroll
+  for (int w = 0; w < NWAVE; ++w) {
+    if constexpr (NP == 1) {
+      x[w] = part[0][w];
+    } else {
+      float sum = part[0][w] + (NP == 3 ? part[1][w] + part[NP - 1][w] : part[1][w]);
+      asm("" : "+v"(sum));
+      x[w] = __builtin_isinf(part[0][w]) ? part[0][w] : sum;
     }
   }
-  if (lane == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      L.ml[(wave * G + g) * 2] = m[g];
-      L.ml[(wave * G + g) * 2 + 1] = l[g];
-    }
-  }
+}
+
+// Workgroup epilogue, after the wavefronts have put their states into L (m, l in log2 units, acc
+// un-normalised): merge them, then write out/out_f32/lse (one split) or the split partials.
+template <int D, int G, bool LOAD_V, int NP>
+__device__ __forceinline__ void finish_merge(const AttnP& p, int b, int h, int split, const MergeLds<D, G, NP>& L,
+                                             bool plain) {
+  const int tid = threadIdx.x;
   __syncthreads();
   const int S = p.num_splits;
   const int64_t hq0 = static_cast<int64_t>(b) * p.Hq + static_cast<int64_t>(h) * G;
   if constexpr (LOAD_V) {
     for (int o = tid; o < G * D; o += NT) {
       const int g = o / D, d = o % D;
-      float A = 0.f, Ls = 0.f;
+      float A = 0.f, Ls = 0.f, x[NWAVE];
+      merged_acc(x, L, g, d);
       if (plain) {
 #pragma unroll
-        for (int w = 0; w < NWAVE; ++w) A += L.acc[(w * G + g) * D + d];
+        for (int w = 0; w < NWAVE; ++w) A += x[w];
         Ls = 1.f;
       } else {
         float M = NEG_INF;
@@ -475,7 +491,7 @@ __device__ __forceinline__ void finish(const AttnP& p, float (&m)[G], float (&l)
         for (int w = 0; w < NWAVE; ++w) {
           const float f = fexp2(L.ml[(w * G + g) * 2] - mu);
           Ls += L.ml[(w * G + g) * 2 + 1] * f;
-          A += L.acc[(w * G + g) * D + d] * f;
+          A += x[w] * f;
         }
       }
       const int64_t hq = hq0 + g;
@@ -504,6 +520,31 @@ __device__ __forceinline__ void finish(const AttnP& p, float (&m)[G], float (&l)
       p.part_ml[(hq * S + split) * 2 + 1] = Ls;
     }
   }
+}
+
+// The VALU engine's wavefront state into L (acc[g][8]: every lane's rows), then the merge.
+template <int D, int G, bool LOAD_V>
+__device__ __forceinline__ void finish(const AttnP& p, float (&m)[G], float (&l)[G], float (&acc)[G][8], int b,
+                                       int h, int split, MergeLds<D, G, LOAD_V ? 1 : 0>& L, bool plain) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  constexpr int VLPR = Lay<D>::VLPR;
+  if constexpr (LOAD_V) {
+    reduce_acc_rows<D, G>(acc);
+    if (lane < VLPR) {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) L.acc[(wave * G + g) * D + 8 * lane + e] = acc[g][e];
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      L.ml[(wave * G + g) * 2] = m[g];
+      L.ml[(wave * G + g) * 2 + 1] = l[g];
+    }
+  }
+  finish_merge<D, G, LOAD_V>(p, b, h, split, L, plain);
 }
 
 template <int D, int G>
@@ -543,31 +584,62 @@ __device__ __forceinline__ void block_softmax(const float (&s)[8][G], int g, flo
 }
 
 
-// ---------------------------------------------------------------- MFMA QK engine
+// ---------------------------------------------------------------- MFMA engine
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 template <int D>
 struct MLay {
-  static constexpr int KS = D / 32;  // 32-dim k-steps of v_mfma_f32_16x16x32_bf16
+  static constexpr int KS = D / 32;   // 32-dim k-steps of v_mfma_f32_16x16x32_bf16
+  static constexpr int VD = D / 16;   // output dims per column of a P V product
+  static constexpr int VN = BLK * D / (WAVE * 8);  // 16-byte V loads per lane and block
 };
 
-// Sum / max over the 16 lanes of each DPP row (every lane gets the row result).
-__device__ __forceinline__ float row16_sum(float v) {
-  v += dpp<DPP_XOR1>(v);
-  v += dpp<DPP_XOR2>(v);
-  v += dpp<DPP_HALF_MIRROR>(v);
-  return v + dpp<DPP_MIRROR>(v);
+// Token of score s[nt][i] on a lane with j4 = lane / 16: four consecutive tokens per lane (fp16 P is
+// written and read in 8-byte pieces).
+__device__ __forceinline__ int mf_tok(int nt, int i, int j4) { return 16 * nt + 4 * j4 + i; }
+
+// Byte offset of this lane's K row within a 16-token tile (row lane % 16 of the A operand) and its
+// 16-byte chunk lane / 16.
+__device__ __forceinline__ uint32_t mf_koff(int lane, int64_t k_st) {
+  return static_cast<uint32_t>((lane & 15) * k_st * 2 + 16 * (lane >> 4));
 }
-__device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, dpp<DPP_XOR1>(v));
-  v = fmaxf(v, dpp<DPP_XOR2>(v));
-  v = fmaxf(v, dpp<DPP_HALF_MIRROR>(v));
-  return fmaxf(v, dpp<DPP_MIRROR>(v));
+// V loads are 16 bytes (8 dims) per lane. D 128: a 16-lane group loads one row, load 4 nt + i the rows
+// mf_tok(nt, i, lane / 16), and column c holds dims 8 c .. + 7. D 64: a group loads two rows, load
+// 2 nt + i the tokens mf_tok(nt, 2 i, lane / 16) (lanes c < 8) and mf_tok(nt, 2 i + 1, ..) (c >= 8);
+// the lanes c and c ^ 8 then exchange halves (v_rows), so that column c holds four dims of both rows:
+// 8 (c % 8) .. + 3, or + 4 .. + 7 for c >= 8. (8-byte loads of one row per group instead: B 16 at 20k,
+// 106 -> 109 us per op.)
+template <int D>
+__device__ __forceinline__ uint32_t mf_voff(int lane, int64_t v_st) {
+  const int j4 = lane >> 4, c = lane & 15;
+  return D == 128 ? static_cast<uint32_t>(4 * j4 * v_st * 2 + 16 * c)
+                  : static_cast<uint32_t>((4 * j4 + (c >> 3)) * v_st * 2 + 16 * (c & 7));
+}
+// First output dim of column c; its VD dims follow.
+template <int D>
+__device__ __forceinline__ int mf_vdim(int c) {
+  return D == 128 ? 8 * c : 8 * (c & 7) + 4 * (c >> 3);
 }
 
-// B operand (K^T) of one 64-token block: kr[nt][kk] = 16 bytes of row t0 + 16 nt + lane%16 at
-// 16-byte chunk 4 kk + lane/16. koffm = (lane % 16) * k_st * 2 + 16 * (lane / 16).
+// Reductions over the four lanes that hold one head's other tokens (lane ^ 16, ^ 32).
+__device__ __forceinline__ float swap_max(float v) {
+  const uint32_t a = __float_as_uint(v);
+  const u32x2 r = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const uint32_t m = __float_as_uint(fmaxf(__uint_as_float(r.x), __uint_as_float(r.y)));
+  const u32x2 t = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+  return fmaxf(__uint_as_float(t.x), __uint_as_float(t.y));
+}
+__device__ __forceinline__ float swap_sum(float v) {
+  const uint32_t a = __float_as_uint(v);
+  const u32x2 r = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const uint32_t m = __float_as_uint(__uint_as_float(r.x) + __uint_as_float(r.y));
+  const u32x2 t = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+  return __uint_as_float(t.x) + __uint_as_float(t.y);
+}
+
+// A operand (K) of one 64-token block: kr[nt][kk] = 16 bytes of this lane's row of tile nt at 16-byte
+// chunk 4 kk + lane/16. koffm = mf_koff.
 template <int D>
 __device__ __forceinline__ void load_k_block_mf(u32x4 (&kr)[4][MLay<D>::KS], rsrc_t rk, uint32_t koffm,
                                                 int64_t k_st, int t0) {
@@ -580,33 +652,246 @@ __device__ __forceinline__ void load_k_block_mf(u32x4 (&kr)[4][MLay<D>::KS], rsr
   }
 }
 
-// A operand (Q): lane (j, c = lane%16) holds head c's dims of chunk 4 kk + j (zero for c >= G).
-template <int D, int G>
-__device__ __forceinline__ void load_q_mf(u32x4 (&qa)[MLay<D>::KS], const AttnP& p, int b, int h, int lane) {
-  const int c = lane & 15, j = lane >> 4;
-  const uint16_t* qp = p.q + b * p.q_sb + (static_cast<int64_t>(h) * G + c) * p.q_sh + 8 * j;
+// V of one 64-token block. voffm = mf_voff.
+template <int D>
+__device__ __forceinline__ void load_v_block_mf(u32x4 (&vr)[MLay<D>::VN], rsrc_t rv, uint32_t voffm, int64_t v_st,
+                                                int t0) {
+  const uint32_t rowb = static_cast<uint32_t>(v_st * 2);
 #pragma unroll
-  for (int kk = 0; kk < MLay<D>::KS; ++kk) qa[kk] = c < G ? ld16(qp + 32 * kk) : u32x4{0u, 0u, 0u, 0u};
+  for (int r = 0; r < MLay<D>::VN; ++r) {
+    const int t = D == 128 ? mf_tok(r / 4, r % 4, 0) : mf_tok(r / 2, 2 * (r % 2), 0);
+    vr[r] = bload16<BUF_NT>(rv, voffm, static_cast<uint32_t>(t0 + t) * rowb);
+  }
 }
 
-// Scores of one block in log2 units, MFMA layout: s[nt][i] = head 4*(lane/16) + i, token
-// t0 + 16 nt + lane%16; tokens >= t_lim masked to -inf.
+// Dwords d (dims 2 d, 2 d + 1 of this lane's column) of tokens (nt, i) and (nt, i + 1), i even.
+template <int D>
+__device__ __forceinline__ void v_pair(const u32x4 (&vr)[MLay<D>::VN], int nt, int i, int d, bool up, uint32_t& a,
+                                       uint32_t& c) {
+  if constexpr (D == 128) {
+    a = vr[4 * nt + i][d];
+    c = vr[4 * nt + i + 1][d];
+  } else {  // up: lanes c >= 8, which loaded the second token's row
+    const u32x4 x = vr[2 * nt + i / 2];
+    const uint32_t other = dppu<DPP_ROR8>(up ? x[d] : x[2 + d]);
+    a = up ? other : x[d];
+    c = up ? x[2 + d] : other;
+  }
+}
+
+// B operand (Q^T): lane (j = lane / 16, c = lane % 16) holds head c % gpad's dims of chunk 4 kk + j
+// (zero past G): every group of gpad columns repeats the group's heads.
+template <int D, int G>
+__device__ __forceinline__ void load_q_mf(u32x4 (&qb)[MLay<D>::KS], const AttnP& p, int b, int h, int lane) {
+  const int c = (lane & 15) % gpad<G>(), j = lane >> 4;
+  const uint16_t* qp = p.q + b * p.q_sb + (static_cast<int64_t>(h) * G + c) * p.q_sh + 8 * j;
+#pragma unroll
+  for (int kk = 0; kk < MLay<D>::KS; ++kk) qb[kk] = c < G ? ld16(qp + 32 * kk) : u32x4{0u, 0u, 0u, 0u};
+}
+
+// Scores of one block in log2 units: s[nt][i] = head (lane % 16) % gpad, token t0 + mf_tok(nt, i,
+// lane / 16); tokens >= t_lim masked to -inf (only the block that t_lim cuts tests them).
 template <int D>
 __device__ __forceinline__ void qk_block_mf(float (&s)[4][4], const u32x4 (&kr)[4][MLay<D>::KS],
-                                            const u32x4 (&qa)[MLay<D>::KS], float scale_log2, int t0, int t_lim,
+                                            const u32x4 (&qb)[MLay<D>::KS], float scale_log2, int t0, int t_lim,
                                             int lane) {
-  const int c = lane & 15;
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
     f32x4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < MLay<D>::KS; ++kk)
-      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, qa[kk]),
-                                                  __builtin_bit_cast(bf16x8_t, kr[nt][kk]), a, 0, 0, 0);
-    const bool ok = t0 + 16 * nt + c < t_lim;
+      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[nt][kk]),
+                                                  __builtin_bit_cast(bf16x8_t, qb[kk]), a, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s[nt][i] = ok ? a[i] * scale_log2 : NEG_INF;
+    for (int i = 0; i < 4; ++i) s[nt][i] = a[i] * scale_log2;
   }
+  if (t0 + BLK > t_lim) {  // uniform
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (t0 + mf_tok(nt, i, lane >> 4) >= t_lim) s[nt][i] = NEG_INF;
+  }
+}
+
+// One block's maximum of a lane's head.
+__device__ __forceinline__ float block_max_mf(const float (&s)[4][4]) {
+  float x = s[0][0];
+#pragma unroll
+  for (int t = 1; t < 16; ++t) x = fmaxf(x, s[t / 4][t % 4]);
+  return swap_max(x);
+}
+
+// e = 2^(s - mt) (mt the block's maximum; 0 where it is -inf) and their sum over the block.
+__device__ __forceinline__ float block_exp_mf(float (&e)[4][4], const float (&s)[4][4], float mt) {
+  const float mtu = mt == NEG_INF ? 0.f : mt;
+  float r[4];
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[nt][i] = fexp2(s[nt][i] - mtu);
+    r[nt] = (e[nt][0] + e[nt][1]) + (e[nt][2] + e[nt][3]);
+  }
+  return swap_sum((r[0] + r[1]) + (r[2] + r[3]));
+}
+
+// Weights of one block as A operands of P V: k-step s covers tiles 2 s and 2 s + 1, element e of lane
+// (c, j4) is the weight of s[2 s + e / 4][e % 4]. Row c is part c / gpad of head c % gpad, and the sum of
+// a head's rows is its result; the parts are bf16 and sum to the fp32 weight (or to the product it was
+// rounded from, where the compiler contracts).
+//   4-head groups   one product, parts (hi, mid, lo, 0): the weight's top 8 significant bits, the next 8
+//                   and the rest, each by truncation.
+//   8-head groups   two products into the same accumulators, parts (hi, mid) then (lo / 2, lo / 2), cut one
+//                   bit lower so that no part of a weight > 0 is 0 (see sat_dec).
+// An infinite V entry meets a part that is 0 only where the weight is 0, or (4-head groups) in rows that
+// merged_acc leaves out then, so it gives the infinity that an fp32 product gives and no NaN.
+// Measured against P through LDS and P V as fp32 FMAs (G x 128 per lane and block at D 128, and 128
+// conversions; op, us, graph-replayed): B 1 at 32k 26.6 -> 25.9 dense, 16.3 -> 14.9 masked with statistics
+// (35% listed); 7 heads, B 6 at 9k, 27.6 -> 24.7; 8 heads, B 4 at 16k, 48.6 -> 45.8; D 64 at 4k 8.7 -> 7.6;
+// B 8 at 32k 156.6 -> 155.0. The loads bound all of these; what went is arithmetic that nothing covered.
+template <int G>
+struct PFrag {
+  static constexpr int NX = gpad<G>() == 8 ? 2 : 1;  // products per k-step
+  static constexpr int NP = gpad<G>() == 8 ? 2 : 3;  // parts (row groups) of a result
+  u32x4 x[NX][2];
+};
+
+// Two values' high halves (bf16 by truncation), the first in the low half.
+__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+constexpr uint32_t BF_HI = 0xffff0000u;
+// The largest float below a (a > 0; 0 stays 0): truncated to bf16 it is below a by at most 2 ulps of bf16
+// and above 0, and a less it is exact and above 0.
+__device__ __forceinline__ uint32_t sat_dec(uint32_t a) { return __builtin_elementwise_sub_sat(a, 1u); }
+
+// The lane's column gives weight 0 where this is false (the unused fourth part of 4-head groups).
+template <int G>
+__device__ __forceinline__ bool part_used(int lane) {
+  return gpad<G>() == 8 || (lane & 15) < 12;
+}
+
+template <int G>
+__device__ __forceinline__ PFrag<G> make_frag(const float (&w)[4][4], int lane) {
+  PFrag<G> f;
+  const int part = (lane & 15) / gpad<G>();
+  const uint32_t m1 = part >= 1 ? BF_HI : 0u, m2 = part >= 2 ? BF_HI : 0u;
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      uint32_t v[2], lo[2];
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        const float a = w[2 * s + u / 2][2 * (u % 2) + o];
+        if constexpr (gpad<G>() == 8) {
+          const uint32_t h = sat_dec(__float_as_uint(a));
+          const float r = a - __uint_as_float(h & BF_HI);
+          const uint32_t m = sat_dec(__float_as_uint(r));
+          v[o] = part != 0 ? m : h;
+          lo[o] = __float_as_uint(0.5f * (r - __uint_as_float(m & BF_HI)));
+        } else {
+          const float r = a - __uint_as_float(__float_as_uint(a) & m1);
+          v[o] = __float_as_uint(r - __uint_as_float(__float_as_uint(r) & m2));
+        }
+      }
+      f.x[0][s][u] = pack_hi(v[0], v[1]);
+      if constexpr (gpad<G>() == 8) f.x[PFrag<G>::NX - 1][s][u] = pack_hi(lo[0], lo[1]);
+    }
+  return f;
+}
+
+// Accumulators of P V: a[j] on lane (c, j4) holds rows 4 j4 + i (part and head as PFrag's rows) of dim
+// mf_vdim(c) + j.
+template <int D, int G>
+struct PVAcc {
+  f32x4_t a[MLay<D>::VD];
+};
+
+template <int D, int G>
+__device__ __forceinline__ void zero_acc(PVAcc<D, G>& acc) {
+#pragma unroll
+  for (int j = 0; j < MLay<D>::VD; ++j) acc.a[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
+
+// acc *= alpha of each row's head (alpha: this lane's head's; row r of a lane's accumulators is head
+// r % gpad, found on lane r % gpad of every 16-lane row).
+template <int D, int G>
+__device__ __forceinline__ void rescale_acc(PVAcc<D, G>& acc, float alpha, int lane) {
+  float al[4];
+  al[0] = dpp<0x150>(alpha);  // row_newbcast
+  al[1] = dpp<0x151>(alpha);
+  al[2] = dpp<0x152>(alpha);
+  al[3] = dpp<0x153>(alpha);
+  if constexpr (gpad<G>() == 8) {
+    const bool up = (lane & 16) != 0;  // rows 4 .. 7 of an 8-row part
+    al[0] = up ? dpp<0x154>(alpha) : al[0];
+    al[1] = up ? dpp<0x155>(alpha) : al[1];
+    al[2] = up ? dpp<0x156>(alpha) : al[2];
+    al[3] = up ? dpp<0x157>(alpha) : al[3];
+  }
+#pragma unroll
+  for (int j = 0; j < MLay<D>::VD; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc.a[j][i] *= al[i];
+}
+
+// acc += P V of one block.
+template <int D, int G>
+__device__ __forceinline__ void pv_block_mf(PVAcc<D, G>& acc, const u32x4 (&vr)[MLay<D>::VN], const PFrag<G>& f,
+                                            int lane) {
+  const bool up = (lane & 8) != 0;
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int d = 0; d < MLay<D>::VD / 2; ++d) {
+      u32x4 lo, hi;  // dims 2 d and 2 d + 1 of this lane's: tokens in pairs
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        uint32_t a, c;
+        v_pair<D>(vr, 2 * s + u / 2, 2 * (u % 2), d, up, a, c);
+        lo[u] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+        hi[u] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+      }
+#pragma unroll
+      for (int n = 0; n < PFrag<G>::NX; ++n) {
+        const bf16x8_t w = __builtin_bit_cast(bf16x8_t, f.x[n][s]);
+        acc.a[2 * d] =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8_t, lo), acc.a[2 * d], 0, 0, 0);
+        acc.a[2 * d + 1] =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8_t, hi), acc.a[2 * d + 1], 0, 0, 0);
+      }
+    }
+}
+
+// The MFMA engine's wavefront state into L (m, l: this lane's head's), then the merge.
+template <int D, int G, bool LOAD_V>
+__device__ __forceinline__ void finish_mf(const AttnP& p, float m, float l, const PVAcc<D, G>& acc, int b, int h,
+                                          int split, MergeLds<D, G, LOAD_V ? PFrag<G>::NP : 0>& L, bool plain) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  const int j4 = lane >> 4, c16 = lane & 15;
+  if constexpr (LOAD_V) {
+    constexpr int VD = MLay<D>::VD, GP = gpad<G>(), NP = PFrag<G>::NP;
+    const int part = 4 * j4 / GP;  // rows 4 j4 .. + 3
+    if (part < NP) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int g = (4 * j4) % GP + i;
+        if (g < G) {
+          float* a = L.acc + ((wave * NP + part) * G + g) * D + mf_vdim<D>(c16);
+#pragma unroll
+          for (int j = 0; j < VD; j += 4)
+            *reinterpret_cast<float4*>(a + j) =
+                make_float4(acc.a[j][i], acc.a[j + 1][i], acc.a[j + 2][i], acc.a[j + 3][i]);
+        }
+      }
+    }
+  }
+  if (lane < G) {
+    L.ml[(wave * G + lane) * 2] = m;
+    L.ml[(wave * G + lane) * 2 + 1] = l;
+  }
+  finish_merge<D, G, LOAD_V>(p, b, h, split, L, plain);
 }
 
 // Split merge: workgroup (b*Hq + hq, 32-dim slice), 256 threads = 8 split classes x 32 dims.

@@ -28,13 +28,17 @@ template <int G, class List>
 __device__ void write_gap_stats(const AttnP& p, const List& list, int n_items, int i0, int n, int split,
                                 int64_t hq0, int wave, int lane, int prev0, int cur0) {
   // blocks a .. a + len - 1, thread t of a team of `stride`: blocks over the team, the G heads in an
-  // unrolled loop (no division by the run-time length)
+  // unrolled loop (no division by the run-time length), through buffer resources (one offset per lane,
+  // the head in the scalar offset; as 64-bit addresses the stores of all heads spilled 88 registers of
+  // the G 4 pass)
+  const uint32_t nb4 = 4u * static_cast<uint32_t>(p.nb);
+  const rsrc_t rs_max = make_rsrc(p.blk_max + hq0 * p.nb, G * nb4), rs_sum = make_rsrc(p.blk_sum + hq0 * p.nb, G * nb4);
   auto put_range = [&](int a, int len, int t, int stride) {
     for (int x = t; x < len; x += stride) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        p.blk_max[(hq0 + g) * p.nb + a + x] = NEG_INF;
-        p.blk_sum[(hq0 + g) * p.nb + a + x] = 0.f;
+        bstore_f32(NEG_INF, rs_max, 4u * static_cast<uint32_t>(a + x), g * nb4);
+        bstore_f32(0.f, rs_sum, 4u * static_cast<uint32_t>(a + x), g * nb4);
       }
     }
   };
@@ -302,12 +306,10 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
   static_assert(!PLANNED || MASKED, "a planned pass is masked");
   static_assert(!(PLANNED && RAG && PAGED), "a planned ragged pass reads a contiguous cache");
   static_assert(!PAGED || MF, "a paged cache is read by the MFMA engine");
-  constexpr int GP = gpad<G>();
-  __shared__ __attribute__((aligned(16))) float sP[NWAVE][BLK * GP];
-  __shared__ __attribute__((aligned(16))) MergeLds<D, G> sL;
+  constexpr int NP = LOAD_V ? (MF ? PFrag<G>::NP : 1) : 0;
+  __shared__ __attribute__((aligned(16))) MergeLds<D, G, NP> sL;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
-  const int r8 = lane >> 3, sub = lane & 7;
 
   // This workgroup's work: (b, KV head h, split) and list positions / blocks [i0, i0 + n) of the
   // n_items of (b, h); Tb, nbb: the sequence's tokens and blocks.
@@ -425,7 +427,8 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     // B 8 172.9 -> 171.4 us per layer-step, config 5's dense pass 111.9 -> 111.3), or of C items
     // and a partial last over all lists of a queued grid (global_lookup's order takes the partial
     // chunks last) or of groups over 4 (config 5's loop 125.1 -> 126.6 cut near-equal).
-    if (global && (G > 4 || grid_queued(p))) {
+    // One sequence is cut into chunks of C too, as the planned pass cuts it (the same result bit for bit).
+    if ((global && (G > 4 || grid_queued(p))) || p.B == 1) {
       i0 = chunk * C;
       n = min(n_items, i0 + C) - i0;
     } else {
@@ -472,15 +475,7 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
 
   const rsrc_t rk = make_rsrc(p.k + b * p.k_sb + h * p.k_sh, head_bytes(Tb, p.k_st, D));
   const rsrc_t rv = make_rsrc(p.v + b * p.v_sb + h * p.v_sh, LOAD_V ? head_bytes(Tb, p.v_st, D) : 0);
-  const uint32_t voff = static_cast<uint32_t>((lane / Lay<D>::VLPR) * p.v_st * 2 + 16 * (lane % Lay<D>::VLPR));
   const int64_t hq0 = static_cast<int64_t>(b) * p.Hq + static_cast<int64_t>(h) * G;
-
-  float acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
-  float* sPw = sP[wave];
 
   // List entry of this wavefront's k-th item (k clamped to its items): a vector load whose value is
   // used two items later, so that waiting for it never waits for the block loads issued after it.
@@ -490,86 +485,71 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     const int blk = __builtin_amdgcn_readfirstlane(MASKED ? e : i0 + wave + NWAVE * k);
     return (blk >= 0 && blk < nbb) ? blk : -1;
   };
-  auto accumulate = [&](const u32x4 (&vr)[Lay<D>::VN], const float (&alpha)[G]) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[g][e] *= alpha[g];
-    pv_block<D, G>(acc, vr, sPw, lane);
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  float m[G], l[G];
   if constexpr (MF) {
-    // ---- MFMA engine: K(j) and V(j) both prefetched one block ahead.
+    // ---- MFMA engine: K(j + 1) is requested after the scores of block j, V(j + 1) after its P V.
     constexpr int KS = MLay<D>::KS;
-    constexpr int NI = G < 4 ? G : 4;               // score rows i in use per lane group
     const int j4 = lane >> 4, c16 = lane & 15;
-    const uint32_t koffm = static_cast<uint32_t>(c16 * p.k_st * 2 + 16 * j4);
+    const uint32_t koffm = mf_koff(lane, p.k_st), voffm = mf_voff<D>(lane, p.v_st);
     // statistics and P of this (b, KV head) through buffer resources: one 32-bit offset per lane
-    // (head 4 j4 + i: + i * row bytes), the block in the scalar offset
+    // (head c16: + c16 row bytes), the block in the scalar offset; out of range past the heads
     const uint32_t nb4 = 4u * static_cast<uint32_t>(p.nb), tp2 = 2u * static_cast<uint32_t>(p.t_pad);
     const rsrc_t rs_max = make_rsrc(STATS ? p.blk_max + hq0 * p.nb : nullptr, STATS ? G * nb4 : 0);
     const rsrc_t rs_sum = make_rsrc(STATS ? p.blk_sum + hq0 * p.nb : nullptr, STATS ? G * nb4 : 0);
     const rsrc_t rs_p = make_rsrc(STATS && p.p_out != nullptr ? p.p_out + hq0 * p.t_pad : nullptr,
                                   STATS && p.p_out != nullptr ? G * tp2 : 0);
-    const uint32_t v_stat = 4u * j4 * nb4, v_p = 4u * j4 * tp2 + 2u * c16;
-    u32x4 qa[KS];
-    load_q_mf<D, G>(qa, p, b, h, lane);
-    float mr[4], lr[4];                             // running (m, l) of head 4 j4 + i
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      mr[i] = NEG_INF;
-      lr[i] = 0.f;
-    }
-    // block blk's scores (tokens >= lim masked: lim = Tb, or 0 for an empty block), statistics and P
-    auto process = [&](int blk, int lim, const u32x4 (&kr)[4][KS], float (&alpha)[G]) {
+    const uint32_t v_stat = c16 * nb4, v_p = c16 * tp2 + 8u * j4;
+    u32x4 qb[KS];
+    load_q_mf<D, G>(qb, p, b, h, lane);
+    float mr = NEG_INF, lr = 0.f;  // running (m, l) of this lane's head c16 % gpad
+    PVAcc<D, G> acc;
+    if constexpr (LOAD_V) zero_acc(acc);
+    // block blk's scores (tokens >= lim masked: lim = Tb, or 0 for an empty block), statistics and P;
+    // pf: its weights, alpha: the accumulators' rescale (this lane's head's). next_k: the K loads of the
+    // block after it, into the registers its scores have just left. (Issued after the softmax: B 8 at 32k
+    // 157.9 against 155.0 us per op; after P V: 159.7.)
+    auto process = [&](int blk, int lim, const u32x4 (&kr)[4][KS], PFrag<G>& pf, float& alpha, auto&& next_k) {
       const int t0 = blk >= 0 ? blk * BLK : 0;
-      float s[4][4];
-      qk_block_mf<D>(s, kr, qa, p.scale_log2, t0, lim, lane);
-      float pv[4][4], ar[4];
+      float s[4][4], e[4][4];
+      qk_block_mf<D>(s, kr, qb, p.scale_log2, t0, lim, lane);
+      __builtin_amdgcn_sched_barrier(0);
+      next_k();
+      __builtin_amdgcn_sched_barrier(0);
+      const float mt = block_max_mf(s);
+      const float st = block_exp_mf(e, s, mt);
+      const float m_new = fmaxf(mr, mt);
+      const float mu = m_new == NEG_INF ? 0.f : m_new;
+      alpha = fexp2(mr - mu);
+      float cf = mt == NEG_INF ? 0.f : fexp2(mt - mu);
+      lr = lr * alpha + st * cf;
+      mr = m_new;
+      if constexpr (STATS) {
+        if (blk >= 0 && c16 < G) {
+          if (j4 == 0) {
+            bstore_f32(mt * LN2, rs_max, v_stat, 4 * blk);
+            bstore_f32(st, rs_sum, v_stat, 4 * blk);
+          }
+          if (p.p_out != nullptr) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int g = 4 * j4 + i;
-        const float mt = row16_max(fmaxf(fmaxf(s[0][i], s[1][i]), fmaxf(s[2][i], s[3][i])));
-        const float mtu = mt == NEG_INF ? 0.f : mt;
-        float e[4];
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) e[nt] = fexp2(s[nt][i] - mtu);
-        const float st = row16_sum((e[0] + e[1]) + (e[2] + e[3]));
-        const float m_new = fmaxf(mr[i], mt);
-        const float mu = m_new == NEG_INF ? 0.f : m_new;
-        ar[i] = fexp2(mr[i] - mu);
-        const float cf = mt == NEG_INF ? 0.f : fexp2(mt - mu);
-        lr[i] = lr[i] * ar[i] + st * cf;
-        mr[i] = m_new;
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) pv[nt][i] = e[nt] * cf;
-        if constexpr (STATS) {
-          if (blk >= 0 && g < G) {
-            if (c16 == 0) {
-              bstore_f32(mt * LN2, rs_max, v_stat + i * nb4, 4 * blk);
-              bstore_f32(st, rs_sum, v_stat + i * nb4, 4 * blk);
-            }
-            if (p.p_out != nullptr) {
-#pragma unroll
-              for (int nt = 0; nt < 4; ++nt) bstore_u16(f2h(e[nt]), rs_p, v_p + i * tp2 + 32 * nt, 2 * t0);
+            for (int nt = 0; nt < 4; ++nt) {
+              bstore_b64(u32x2{f2h(e[nt][0]) | static_cast<uint32_t>(f2h(e[nt][1])) << 16,
+                               f2h(e[nt][2]) | static_cast<uint32_t>(f2h(e[nt][3])) << 16},
+                         rs_p, v_p + 32 * nt, 2 * t0);
             }
           }
         }
       }
       if constexpr (LOAD_V) {
-        if (4 * j4 < GP) {
+        cf = part_used<G>(lane) ? cf : 0.f;
 #pragma unroll
-          for (int nt = 0; nt < 4; ++nt)
-            *reinterpret_cast<float4*>(sPw + (16 * nt + c16) * GP + 4 * j4) =
-                make_float4(pv[nt][0], NI > 1 ? pv[nt][1] : 0.f, NI > 2 ? pv[nt][2] : 0.f, NI > 3 ? pv[nt][3] : 0.f);
-        }
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) e[nt][i] *= cf;
+        pf = make_frag<G>(e, lane);
       }
-#pragma unroll
-      for (int g = 0; g < G; ++g) alpha[g] = lane_value(ar[g % 4], 16 * (g / 4));
+    };
+    auto accumulate = [&](const u32x4 (&vr)[MLay<D>::VN], const PFrag<G>& pf, float alpha) {
+      rescale_acc<D, G>(acc, alpha, lane);
+      pv_block_mf<D, G>(acc, vr, pf, lane);
     };
     if (nw > 0 && !LOAD_V && PAGED) {
       // K only over a paged cache: two blocks in flight as below, each through its page's resource
@@ -589,8 +569,9 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
                            max(bld, 0) * BLK);
         __builtin_amdgcn_sched_barrier(0);
         if (k < nw) {
-          float alpha[G];
-          process(bac, (bac >= 0 && gac >= 0) ? Tb : 0, ac, alpha);
+          PFrag<G> pf;
+          float alpha;
+          process(bac, (bac >= 0 && gac >= 0) ? Tb : 0, ac, pf, alpha, [] {});
         }
         __builtin_amdgcn_sched_barrier(0);
       };
@@ -614,8 +595,9 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         load_k_block_mf<D>(ld, rk, koffm, p.k_st, (k + 1 < nw ? max(bld, 0) : nbb) * BLK);
         __builtin_amdgcn_sched_barrier(0);
         if (k < nw) {
-          float alpha[G];
-          process(bac, bac >= 0 ? Tb : 0, ac, alpha);
+          PFrag<G> pf;
+          float alpha;
+          process(bac, bac >= 0 ? Tb : 0, ac, pf, alpha, [] {});
         }
         __builtin_amdgcn_sched_barrier(0);
       };
@@ -628,7 +610,7 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
       // beyond), an empty block's spans nothing; both are built before the block ahead is scored
       // (built after it, the compiler spilled the freshly loaded K block)
       u32x4 kr[4][KS];
-      u32x4 vr[Lay<D>::VN];
+      u32x4 vr[MLay<D>::VN];
       auto page_rsrc = [&](const uint16_t* pool, int64_t psb, int64_t sh, int64_t st, int blk, int pg) {
         return block_rsrc(pool, psb, sh, st, h, blk, pg, Tb, D);
       };
@@ -636,60 +618,71 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
       int blk, pg;
       paged_item(0, blk, pg);
       load_k_block_mf<D>(kr, page_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, blk, pg), koffm, p.k_st, max(blk, 0) * BLK);
-      load_v_block<D>(vr, page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk, pg), voff, p.v_st, max(blk, 0) * BLK);
-      for (int k = 0; k + 1 < nw; ++k) {
-        int blk_n, pg_n;
-        paged_item(k + 1, blk_n, pg_n);
+      __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop: a wait for K is none for V
+      load_v_block_mf<D>(vr, page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk, pg), voffm, p.v_st, max(blk, 0) * BLK);
+      for (int k = 0; k < nw; ++k) {  // past the last item an empty block's loads (zeros, no memory access)
+        int blk_n = -1, pg_n = -1;
+        if (k + 1 < nw) paged_item(k + 1, blk_n, pg_n);
         const rsrc_t rk_n = page_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, blk_n, pg_n);
         const rsrc_t rv_n = page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk_n, pg_n);
-        float alpha[G];
-        process(blk, lim_of(blk, pg), kr, alpha);
+        PFrag<G> pf;
+        float alpha;
+        process(blk, lim_of(blk, pg), kr, pf, alpha,
+                [&] { load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, max(blk_n, 0) * BLK); });
+        accumulate(vr, pf, alpha);
         __builtin_amdgcn_sched_barrier(0);
-        load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, max(blk_n, 0) * BLK);
-        __builtin_amdgcn_sched_barrier(0);
-        accumulate(vr, alpha);
-        __builtin_amdgcn_sched_barrier(0);
-        load_v_block<D>(vr, rv_n, voff, p.v_st, max(blk_n, 0) * BLK);
+        load_v_block_mf<D>(vr, rv_n, voffm, p.v_st, max(blk_n, 0) * BLK);
         blk = blk_n;
         pg = pg_n;
       }
-      float alpha[G];
-      process(blk, lim_of(blk, pg), kr, alpha);
-      accumulate(vr, alpha);
     } else if (nw > 0) {
       u32x4 kr[4][KS];
-      u32x4 vr[Lay<D>::VN];
+      u32x4 vr[MLay<D>::VN];
       int e_n = entry_of(1);
       int blk = block_of(entry_of(0), 0);
       load_k_block_mf<D>(kr, rk, koffm, p.k_st, max(blk, 0) * BLK);
-      if constexpr (LOAD_V) load_v_block<D>(vr, rv, voff, p.v_st, max(blk, 0) * BLK);
-      for (int k = 0; k + 1 < nw; ++k) {
+      __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop: a wait for K is none for V
+      load_v_block_mf<D>(vr, rv, voffm, p.v_st, max(blk, 0) * BLK);
+      // Every step issues the same loads; the last one's read beyond the head's buffer range (zeros, no
+      // memory access). (The last block peeled off the loop, or the loop left in its middle: the
+      // compiler spilled the first block's K and V on the way in, and waited for them there.)
+      for (int k = 0; k < nw; ++k) {
         const int e_nn = entry_of(k + 2);
-        const int blk_n = block_of(e_n, k + 1);
+        const int blk_n = block_of(e_n, min(k + 1, nw - 1));
+        const int t_n = (k + 1 < nw ? max(blk_n, 0) : nbb) * BLK;
         e_n = e_nn;
-        float alpha[G];
-        process(blk, blk >= 0 ? Tb : 0, kr, alpha);
+        PFrag<G> pf;
+        float alpha;
+        process(blk, blk >= 0 ? Tb : 0, kr, pf, alpha, [&] { load_k_block_mf<D>(kr, rk, koffm, p.k_st, t_n); });
+        accumulate(vr, pf, alpha);
         __builtin_amdgcn_sched_barrier(0);
-        load_k_block_mf<D>(kr, rk, koffm, p.k_st, max(blk_n, 0) * BLK);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (LOAD_V) {
-          accumulate(vr, alpha);
-          __builtin_amdgcn_sched_barrier(0);
-          load_v_block<D>(vr, rv, voff, p.v_st, max(blk_n, 0) * BLK);
-        }
+        load_v_block_mf<D>(vr, rv, voffm, p.v_st, t_n);
         blk = blk_n;
       }
-      float alpha[G];
-      process(blk, blk >= 0 ? Tb : 0, kr, alpha);
-      if constexpr (LOAD_V) accumulate(vr, alpha);
     }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      m[g] = lane_value(mr[g % 4], 16 * (g / 4));
-      l[g] = lane_value(lr[g % 4], 16 * (g / 4));
-    }
+    finish_mf<D, G, LOAD_V>(p, mr, lr, acc, b, h, slot_base + split, sL, false);
   } else {
     // ---- VALU engine: V(j) issued after QK(j), together with K(j+1) (register budget).
+    constexpr int GP = gpad<G>();
+    __shared__ __attribute__((aligned(16))) float sP[NWAVE][BLK * GP];
+    float* sPw = sP[wave];
+    const int r8 = lane >> 3, sub = lane & 7;
+    const uint32_t voff = static_cast<uint32_t>((lane / Lay<D>::VLPR) * p.v_st * 2 + 16 * (lane % Lay<D>::VLPR));
+    float m[G], l[G], acc[G][8];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
+    auto accumulate = [&](const u32x4 (&vr)[Lay<D>::VN], const float (&alpha)[G]) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[g][e] *= alpha[g];
+      pv_block<D, G>(acc, vr, sPw, lane);
+      __builtin_amdgcn_wave_barrier();
+    };
     const uint32_t koff = static_cast<uint32_t>(r8 * p.k_st * 2 + 16 * sub);
     u32x4 qv[G][Lay<D>::KC];
     load_q<D, G>(qv, p, b, h, lane);
@@ -753,8 +746,8 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         accumulate(vr, alpha);
       }
     }
+    finish<D, G, LOAD_V>(p, m, l, acc, b, h, slot_base + split, sL, false);
   }
-  finish<D, G, LOAD_V>(p, m, l, acc, b, h, slot_base + split, sL, false);
   if constexpr (MASKED && STATS)
     if (gaps) write_gap_stats<G>(p, list, n_items, i0, n, split, hq0, wave, lane, gap_prev, gap_cur);
   if constexpr (PLANNED) {

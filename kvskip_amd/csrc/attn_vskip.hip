@@ -8,9 +8,9 @@ namespace kvs {
 namespace {
 
 // Single-pass V-skip. Per block: QK -> block log-sum-exp per head (log2 units) -> the
-// group's vote -> only then the V loads of that block; the next block's K loads are issued
-// right after, so V(i) overlaps QK(i+1)'s loads. The softmax update and P of a block are
-// computed as if the block were kept and committed only if the group keeps it.
+// group's vote -> only then the V loads of that block (the VALU engine: the next block's K loads
+// right after them; the softmax update and P of a block computed as if it were kept and committed
+// only if the group keeps it).
 // PAGED (MFMA engine only): K / V in pages of a pool through p.block_table; an invalid page reads as
 // an empty block.
 template <int D, int G, bool MF, bool PAGED = false>
@@ -18,15 +18,13 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
   static_assert(!PAGED || MF, "a paged cache is read by the MFMA engine");
   constexpr int GP = gpad<G>();
   __shared__ int sPg[PAGED ? MAX_NB : 1];
-  __shared__ __attribute__((aligned(16))) float sP[NWAVE][BLK * GP];
-  __shared__ __attribute__((aligned(16))) MergeLds<D, G> sL;
+  __shared__ __attribute__((aligned(16))) MergeLds<D, G, MF ? PFrag<G>::NP : 1> sL;
   __shared__ float sLse0[G];
   __shared__ int sLoaded[NWAVE];
 
   int split, h, b;
   work_coords(p.num_splits, p.Hkv, p.B, split, h, b);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
-  const int r8 = lane >> 3, sub = lane & 7;
   const int nb = p.nb;
   const int per = (nb + p.num_splits - 1) / p.num_splits;
   const int i0 = min(nb, split * per);
@@ -34,42 +32,31 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
   const int nw = n > wave ? (n - wave + NWAVE - 1) / NWAVE : 0;
   const rsrc_t rk = make_rsrc(p.k + b * p.k_sb + h * p.k_sh, head_bytes(p.T, p.k_st, D));
   const rsrc_t rv = make_rsrc(p.v + b * p.v_sb + h * p.v_sh, head_bytes(p.T, p.v_st, D));
-  const uint32_t voff = static_cast<uint32_t>((lane / Lay<D>::VLPR) * p.v_st * 2 + 16 * (lane % Lay<D>::VLPR));
   const int64_t hq0 = static_cast<int64_t>(b) * p.Hq + static_cast<int64_t>(h) * G;
-
-  float acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
-  float* sPw = sP[wave];
   int loaded = 0;
-  float m[G], l[G];
-  u32x4 vr[Lay<D>::VN];
-  auto pv = [&]() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    pv_block<D, G>(acc, vr, sPw, lane);
-    __builtin_amdgcn_wave_barrier();
-  };
 
   if constexpr (MF) {
     constexpr int KS = MLay<D>::KS;
-    constexpr int NI = G < 4 ? G : 4;
     const int j4 = lane >> 4, c16 = lane & 15;
-    const uint32_t koffm = static_cast<uint32_t>(c16 * p.k_st * 2 + 16 * j4);
-    u32x4 qa[KS];
-    load_q_mf<D, G>(qa, p, b, h, lane);
+    const int hd = c16 % GP;  // this lane's head (none from G on)
+    const uint32_t koffm = mf_koff(lane, p.k_st), voffm = mf_voff<D>(lane, p.v_st);
+    u32x4 qb[KS];
+    load_q_mf<D, G>(qb, p, b, h, lane);
     u32x4 kr[4][KS];
+    u32x4 vr[MLay<D>::VN];
+    PVAcc<D, G> acc;
+    zero_acc(acc);
     // paged: block blk's K / V resource (item t's page from LDS) and its token limit (0: empty)
     auto page_at = [&](int t) { return PAGED ? __builtin_amdgcn_readfirstlane(sPg[t]) : 0; };
     auto krs = [&](int blk, int pg) { return PAGED ? block_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, h, blk, pg, p.T, D) : rk; };
     auto vrs = [&](int blk, int pg) { return PAGED ? block_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, h, blk, pg, p.T, D) : rv; };
     auto lim_of = [&](int pg) { return pg >= 0 ? p.T : 0; };
     if constexpr (PAGED) gather_pages(p, b, n, nb, [&](int t) { return i0 + t; }, sPg, nullptr);
-    // normaliser estimate (log2 units) per head: lse_prev, or the block-0 log-sum-exp
+    // normaliser estimate (log2 units) of this lane's head: lse_prev, or the block-0 log-sum-exp (found by
+    // wavefront 0). With lse_prev nothing stands before the first block's loads.
+    float lse0 = 0.f;
     if (p.lse_prev != nullptr) {
-      if (tid < G) sLse0[tid] = p.lse_prev[hq0 + tid] * LOG2E;
+      lse0 = p.lse_prev[hq0 + min(hd, G - 1)] * LOG2E;
     } else if (wave == 0) {
       int pg0 = 0;
       if constexpr (PAGED) {
@@ -77,100 +64,82 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
         if (pg0 < 0 || pg0 >= p.num_pages) pg0 = -1;
       }
       load_k_block_mf<D>(kr, krs(0, pg0), koffm, p.k_st, 0);
-      float s[4][4];
-      qk_block_mf<D>(s, kr, qa, p.scale_log2, 0, lim_of(pg0), lane);
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const float mt = row16_max(fmaxf(fmaxf(s[0][i], s[1][i]), fmaxf(s[2][i], s[3][i])));
-        const float mtu = mt == NEG_INF ? 0.f : mt;  // an empty block 0 (paged): -inf, every block kept
-        float sum = 0.f;
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) sum += fexp2(s[nt][i] - mtu);
-        const float lse0 = mtu + flog2(row16_sum(sum));
-        const int g = 4 * j4 + i;
-        if (c16 == 0 && g < G) sLse0[g] = lse0;
-      }
+      float s[4][4], e[4][4];
+      qk_block_mf<D>(s, kr, qb, p.scale_log2, 0, lim_of(pg0), lane);
+      const float mt = block_max_mf(s);  // an empty block 0 (paged): -inf, every block kept
+      const float sum = block_exp_mf(e, s, mt);
+      if (j4 == 0 && c16 < G) sLse0[c16] = (mt == NEG_INF ? 0.f : mt) + flog2(sum);
     }
-    __syncthreads();
-    float lse0r[4], mr[4], lr[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int g = 4 * j4 + i;
-      lse0r[i] = g < G ? sLse0[g] : 0.f;
-      mr[i] = NEG_INF;
-      lr[i] = 0.f;
+    if (p.lse_prev == nullptr) {
+      __syncthreads();
+      lse0 = sLse0[min(hd, G - 1)];
     }
+    float mr = NEG_INF, lr = 0.f;
+    // Item k of this wavefront is block i0 + wave + 4 k: K of the next item is requested right after the
+    // scores (past the last item beyond the head's range: zeros, no memory access), V only if the group
+    // keeps the block. Measured (op, us; B 8 at 32k nothing kept / 64k peaked): the P V by FMAs and K
+    // requested after the vote 98.3 / 44.6; P V on MFMA 93.9 / 42.2; K requested after the scores 91.8 /
+    // 42.2. V requested always (out of range where not kept) and used a step later: 113.0.
     int pg = nw > 0 ? page_at(wave) : -1;
     if (nw > 0) load_k_block_mf<D>(kr, krs(i0 + wave, pg), koffm, p.k_st, (i0 + wave) * BLK);
     for (int k = 0; k < nw; ++k) {
       const int blk = i0 + wave + NWAVE * k;
-      const int t0 = blk * BLK;
       const bool more = k + 1 < nw;
       // this block's V and the next block's K resources, built before the scores
       const int pg_n = more ? page_at(wave + NWAVE * (k + 1)) : -1;
       const rsrc_t rv_c = vrs(blk, pg), rk_n = krs(blk + NWAVE, pg_n);
-      float s[4][4];
-      qk_block_mf<D>(s, kr, qa, p.scale_log2, t0, lim_of(pg), lane);
+      float s[4][4], e[4][4];
+      qk_block_mf<D>(s, kr, qb, p.scale_log2, blk * BLK, lim_of(pg), lane);
       pg = pg_n;
-      float tm[4], tl[4], ta[4], pv4[4][4];
-      bool vote = false;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int g = 4 * j4 + i;
-        const float mt = row16_max(fmaxf(fmaxf(s[0][i], s[1][i]), fmaxf(s[2][i], s[3][i])));
-        const float mtu = mt == NEG_INF ? 0.f : mt;
-        float e[4];
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) e[nt] = fexp2(s[nt][i] - mtu);
-        const float st = row16_sum((e[0] + e[1]) + (e[2] + e[3]));
-        vote = vote || (g < G && mtu + flog2(st) - lse0r[i] >= p.log2_tau);
-        const float m_new = fmaxf(mr[i], mt);
-        const float mu = m_new == NEG_INF ? 0.f : m_new;
-        ta[i] = fexp2(mr[i] - mu);
-        const float cf = mt == NEG_INF ? 0.f : fexp2(mt - mu);
-        tl[i] = lr[i] * ta[i] + st * cf;
-        tm[i] = m_new;
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) pv4[nt][i] = e[nt] * cf;
-      }
-      // P as if kept (unused otherwise), before any load is issued
-      if (4 * j4 < GP) {
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-          *reinterpret_cast<float4*>(sPw + (16 * nt + c16) * GP + 4 * j4) = make_float4(
-              pv4[nt][0], NI > 1 ? pv4[nt][1] : 0.f, NI > 2 ? pv4[nt][2] : 0.f, NI > 3 ? pv4[nt][3] : 0.f);
-      }
+      __builtin_amdgcn_sched_barrier(0);
+      load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, (PAGED || more ? blk + NWAVE : nb) * BLK);
+      __builtin_amdgcn_sched_barrier(0);
+      const float mt = block_max_mf(s);
+      const float mtu = mt == NEG_INF ? 0.f : mt;
+      const float st = block_exp_mf(e, s, mt);
+      const bool vote = hd < G && mtu + flog2(st) - lse0 >= p.log2_tau;
       const bool need = blk == 0 || blk >= nb - p.local || __ballot(vote) != 0;
       if (p.v_keep != nullptr && lane == 0) p.v_keep[(static_cast<int64_t>(b) * p.Hkv + h) * nb + blk] = need ? 1 : 0;
       __builtin_amdgcn_sched_barrier(0);
       if (need) {
         ++loaded;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          mr[i] = i < NI ? tm[i] : mr[i];
-          lr[i] = i < NI ? tl[i] : lr[i];
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float a = lane_value(ta[g % 4], 16 * (g / 4));
-#pragma unroll
-          for (int u = 0; u < 8; ++u) acc[g][u] *= a;
-        }
+        load_v_block_mf<D>(vr, rv_c, voffm, p.v_st, blk * BLK);
         __builtin_amdgcn_sched_barrier(0);
-        load_v_block<D>(vr, rv_c, voff, p.v_st, t0);
-        if (more) load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, (blk + NWAVE) * BLK);
-        __builtin_amdgcn_sched_barrier(0);
-        pv();
-      } else if (more) {
-        load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, (blk + NWAVE) * BLK);
+        const float m_new = fmaxf(mr, mt);
+        const float mu = m_new == NEG_INF ? 0.f : m_new;
+        const float alpha = fexp2(mr - mu);
+        float cf = mt == NEG_INF ? 0.f : fexp2(mt - mu);
+        lr = lr * alpha + st * cf;
+        mr = m_new;
+        cf = part_used<G>(lane) ? cf : 0.f;
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) e[nt][i] *= cf;
+        const PFrag<G> pf = make_frag<G>(e, lane);
+        rescale_acc<D, G>(acc, alpha, lane);
+        pv_block_mf<D, G>(acc, vr, pf, lane);
       }
     }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      m[g] = lane_value(mr[g % 4], 16 * (g / 4));
-      l[g] = lane_value(lr[g % 4], 16 * (g / 4));
-    }
+    if (lane == 0) sLoaded[wave] = loaded;
+    finish_mf<D, G, true>(p, mr, lr, acc, b, h, split, sL, false);
   } else {
+    __shared__ __attribute__((aligned(16))) float sP[NWAVE][BLK * GP];
+    float* sPw = sP[wave];
+    const int r8 = lane >> 3, sub = lane & 7;
+    const uint32_t voff = static_cast<uint32_t>((lane / Lay<D>::VLPR) * p.v_st * 2 + 16 * (lane % Lay<D>::VLPR));
+    float m[G], l[G], acc[G][8];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
+    u32x4 vr[Lay<D>::VN];
+    auto pv = [&]() {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      pv_block<D, G>(acc, vr, sPw, lane);
+      __builtin_amdgcn_wave_barrier();
+    };
     const uint32_t koff = static_cast<uint32_t>(r8 * p.k_st * 2 + 16 * sub);
     u32x4 qv[G][Lay<D>::KC];
     load_q<D, G>(qv, p, b, h, lane);
@@ -256,9 +225,9 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
         load_k_block<D>(kr, rk, koff, p.k_st, (blk + NWAVE) * BLK);
       }
     }
+    if (lane == 0) sLoaded[wave] = loaded;
+    finish<D, G, true>(p, m, l, acc, b, h, split, sL, false);
   }
-  if (lane == 0) sLoaded[wave] = loaded;
-  finish<D, G, true>(p, m, l, acc, b, h, split, sL, false);
   if (tid == 0 && p.vcount != nullptr) {
     int tot = 0;
 #pragma unroll
@@ -276,30 +245,24 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
 template <int D, int G, bool PAGED, class ListAt, class ScaleAt>
 __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b, int n_items, ListAt list_at,
                                         ScaleAt scale_at) {
-  constexpr int GP = gpad<G>();
   __shared__ int sPg[PAGED ? MAX_NB : 1];
   __shared__ int sBk[PAGED ? MAX_NB : 1];
-  __shared__ __attribute__((aligned(16))) float sP[NWAVE][BLK * GP];
-  __shared__ __attribute__((aligned(16))) MergeLds<D, G> sL;
+  __shared__ __attribute__((aligned(16))) MergeLds<D, G, PFrag<G>::NP> sL;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int per = (n_items + p.num_splits - 1) / p.num_splits;
   const int i0 = min(n_items, split * per);
   const int n = min(n_items, i0 + per) - i0;
   const rsrc_t rv = make_rsrc(p.v + b * p.v_sb + h * p.v_sh, head_bytes(p.T, p.v_st, D));
-  const uint32_t voff = static_cast<uint32_t>((lane / Lay<D>::VLPR) * p.v_st * 2 + 16 * (lane % Lay<D>::VLPR));
+  const uint32_t voffm = mf_voff<D>(lane, p.v_st);
   const int64_t hq0 = static_cast<int64_t>(b) * p.Hq + static_cast<int64_t>(h) * G;
 
-  float m[G], l[G], acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = 0.f;
-    l[g] = 1.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
-  }
-  float* sPw = sP[wave];
-  const int pg = lane >> 3, ppart = lane & 7;  // P staging: head pg, tokens 8*ppart .. +8
+  PVAcc<D, G> acc;
+  zero_acc(acc);
+  // this lane's head and whether its column carries a part of it; its weights are those of tokens
+  // 16 nt + 4 (lane / 16) .. + 3 of a block (mf_tok)
+  const int hd = (lane & 15) % gpad<G>(), g = min(hd, G - 1);
+  const bool used = hd < G && part_used<G>(lane);
   // Items i0 + wave + 4k of this wavefront through a ring of R buffers: V, P and the scale of the
   // next R - 1 items are in flight while item k is accumulated (R = 2: a third buffer measured
   // slower, 21.7 vs 20 us at config 2's shape); list entries are loaded two items before their blocks (waiting for an entry
@@ -313,8 +276,8 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
     return (blk >= 0 && blk < p.nb) ? blk : -1;
   };
   struct Item {
-    u32x4 vr[Lay<D>::VN];
-    u32x4 raw;
+    u32x4 vr[MLay<D>::VN];
+    u32x2 raw[4];
     float f;
   };
   // unconditional: out-of-range entries load block 0; past the last item (blk == PAST) V reads
@@ -323,27 +286,25 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
   auto load = [&](Item& it, int blk, int pgv = -1) {
     const int t0 = max(blk, 0) * BLK;
     if constexpr (PAGED)  // an empty block (blk < 0 or no page) reads zeros
-      load_v_block<D>(it.vr, block_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, h, blk, pgv, p.T, D), voff, p.v_st, t0);
+      load_v_block_mf<D>(it.vr, block_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, h, blk, pgv, p.T, D), voffm, p.v_st, t0);
     else
-      load_v_block<D>(it.vr, rv, voff, p.v_st, blk == PAST ? p.nb * BLK : t0);
-    const int g = pg < G ? pg : 0;
+      load_v_block_mf<D>(it.vr, rv, voffm, p.v_st, blk == PAST ? p.nb * BLK : t0);
     it.f = scale_at(max(blk, 0), g);
-    it.raw = ld16(p.p_in + (hq0 + g) * p.t_pad + t0 + 8 * ppart);
+    const uint16_t* pp = p.p_in + (hq0 + g) * p.t_pad + t0 + 4 * (lane >> 4);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) it.raw[nt] = *reinterpret_cast<const u32x2*>(pp + 16 * nt);
   };
   auto accumulate = [&](const Item& it, int blk) {
     if (blk < 0) return;  // uniform
-    if (pg < G) {
-      const uint32_t w[4] = {it.raw.x, it.raw.y, it.raw.z, it.raw.w};
+    float w[4][4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        sPw[(8 * ppart + 2 * u) * GP + pg] = h2f(static_cast<uint16_t>(w[u] & 0xffffu)) * it.f;
-        sPw[(8 * ppart + 2 * u + 1) * GP + pg] = h2f(static_cast<uint16_t>(w[u] >> 16)) * it.f;
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = h2f(static_cast<uint16_t>(it.raw[nt][i / 2] >> (16 * (i % 2)))) * it.f;
+        w[nt][i] = used ? x : 0.f;
       }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    pv_block<D, G>(acc, it.vr, sPw, lane);
-    __builtin_amdgcn_wave_barrier();
+    pv_block_mf<D, G>(acc, it.vr, make_frag<G>(w, lane), lane);
   };
   if constexpr (PAGED) gather_pages(p, b, n, p.nb, [&](int t) { return list_at(i0 + t); }, sPg, sBk);
   if (PAGED && nw > 0) {
@@ -403,7 +364,7 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
       }
     }
   }
-  finish<D, G, true>(p, m, l, acc, b, h, split, sL, true);
+  finish_mf<D, G, true>(p, 0.f, 1.f, acc, b, h, split, sL, true);
 }
 
 template <int D, int G, bool PAGED = false>

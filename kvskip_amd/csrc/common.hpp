@@ -16,6 +16,7 @@ constexpr float NEG_INF = -__builtin_huge_valf();
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // bf16 pair packed in a dword -> the two fp32 values (exact).
 __device__ __forceinline__ float bf_lo(uint32_t x) { return __uint_as_float(x << 16); }
@@ -168,6 +169,9 @@ __device__ __forceinline__ void bstore_f32(float v, rsrc_t r, uint32_t voff, uin
 }
 __device__ __forceinline__ void bstore_u16(uint16_t v, rsrc_t r, uint32_t voff, uint32_t soff) {
   __builtin_amdgcn_raw_buffer_store_b16(v, r, static_cast<int>(voff), static_cast<int>(soff), 0);
+}
+__device__ __forceinline__ void bstore_b64(u32x2 v, rsrc_t r, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, r, static_cast<int>(voff), static_cast<int>(soff), 0);
 }
 
 // Online log-sum-exp accumulator in natural units (planner): (m, s) with s = sum exp(x - m).
