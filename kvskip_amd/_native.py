@@ -124,6 +124,30 @@ def lib() -> ctypes.CDLL:
     return _LIB
 
 
+# The entry points that the native host module calls, in the order of its table (csrc/host.cpp).
+HOST_CALLS = ("decode", "decode_splits", "merge_splits", "pv", "vskip1", "pv_select", "select", "plan", "plan_scores",
+              "update", "merge_update", "decode_splits_update", "decode_splits_planned", "plan_part_floats", "last_error")
+_HOST = None
+
+
+def host():
+    """The native host module (kvskip_amd/_host.so), bound to the loaded library (raises if either is not built)."""
+    global _HOST
+    if _HOST is None:
+        import torch
+
+        h = lib()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError("kvskip_amd: the native host module kvskip_amd/_host.so is missing or does not load; build it "
+                               "with `python -c 'import __graft_entry__ as g; g.build()'`") from e
+        _host.bind(tuple(ctypes.cast(getattr(h, "kvskip_" + n), c_void_p).value for n in HOST_CALLS),
+                   torch._C._cuda_getCurrentRawStream)
+        _HOST = _host
+    return _HOST
+
+
 def check(rc: int) -> None:
     """Raise RuntimeError with the library's message if rc != 0."""
     if rc != 0:

@@ -17,6 +17,7 @@ free); a block is 64 tokens from position 0; G = Hq / Hkv in {1, 2, 4, 7, 8}; D 
 
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
 
@@ -30,20 +31,18 @@ WG_PER_CU = 1          # attention workgroups (4 wavefronts each) per CU in the 
 
 def ext():
     """The operator module, with the native library loaded (it raises if the library is missing)."""
-    from . import _native
-    _native.lib()
+    _ops._host()
     return _ops
+
+
+@functools.lru_cache(maxsize=None)
+def _device_cus(index: int) -> int:
+    return torch.cuda.get_device_properties(index).multi_processor_count
 
 
 def num_sms() -> int:
     """Compute units of the current device (256 on MI355X)."""
-    return torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
-
-
-def _split_score(bh: int, splits: int, slots: int) -> float:
-    """How fully bh * splits workgroups use whole waves of `slots`, less 0.002 per split."""
-    waves = bh * splits / slots
-    return waves / math.ceil(waves) - 0.002 * splits
+    return _device_cus(torch.cuda.current_device())
 
 
 def num_splits_for(bh: int, n_tiles: int, sms: int | None = None, max_splits: int = 256,
@@ -52,15 +51,7 @@ def num_splits_for(bh: int, n_tiles: int, sms: int | None = None, max_splits: in
     kernels/kvskip.py:51-67: the best wave efficiency over the resident workgroup slots (here CUs x
     WG_PER_CU), 0.002 per split against more splits, every split keeping >= min_tiles blocks; the
     smallest count wins ties."""
-    slots = (sms or num_sms()) * WG_PER_CU
-    most = 1                                       # ceil(n / s) only falls as s grows
-    while most < max_splits and math.ceil(n_tiles / (most + 1)) >= min_tiles:
-        most += 1
-    best = 1
-    for s in range(2, most + 1):
-        if _split_score(bh, s, slots) > _split_score(bh, best, slots) + 1e-9:
-            best = s
-    return best
+    return _ops._host().num_splits(bh, n_tiles, (sms or num_sms()) * WG_PER_CU, max_splits, min_tiles)
 
 
 def ragged_splits(B: int, Hkv: int, nb_max: int, sms: int | None = None, G: int = 4, carry: bool = False) -> int:

@@ -174,27 +174,22 @@ class FusedPlanner:
         dev = q.device
         f32 = dict(dtype=torch.float32, device=dev)
         self.NBC = NBC
-        self.state = dict(
-            csum=torch.zeros(B, Hkv, NBC, D, **f32),
+        BH, heads, qheads = ("i4", (B * Hkv,)), (B, Hkv), (B, Hq)
+        zero = dict(cs_ref=("f4", (*qheads, NBC)), cs_now=("f4", (*qheads, NBC)), keep=("u1", (*heads, NBC)),
+                    lse_att=("f4", qheads), age=("i4", heads), flags=("i4", (Hkv,)), trig=("u1", heads),
+                    block_idx=("i4", (*heads, NBC)), block_cnt=("i4", heads), calib=("f4", heads), est=("f4", heads),
+                    aix=("u1", heads), idx=("u1", (B, NBC)),
+                    tlen=("i4", (B,)),              # this step's lengths (ragged)
+                    lens=("i4", (B,)),              # all T, for batch_balance
+                    ticket=BH)                      # one-launch plan (self-resetting)
+        self.state = dict(zip(zero, E._host().zeroed(tuple(zero.values()), q)))      # one allocation, one fill
+        self.state.update(
+            csum=torch.empty(B, Hkv, NBC, D, **f32),            # block_sums writes every block
             lse_ref=torch.full((B, Hq, NBC), -math.inf, **f32),
-            cs_ref=torch.zeros(B, Hq, NBC, **f32),
-            keep=torch.zeros(B, Hkv, NBC, dtype=torch.uint8, device=dev),
-            lse_att=torch.zeros(B, Hq, **f32),
-            age=torch.zeros(B, Hkv, dtype=torch.int32, device=dev),
-            flags=torch.tensor(self.policy.flags(Hkv), dtype=torch.int32, device=dev),
-            cs_now=torch.zeros(B, Hq, NBC, **f32),
-            trig=torch.zeros(B, Hkv, dtype=torch.uint8, device=dev),
-            block_idx=torch.zeros(B, Hkv, NBC, dtype=torch.int32, device=dev),
-            block_cnt=torch.zeros(B, Hkv, dtype=torch.int32, device=dev),
-            calib=torch.zeros(B, Hkv, **f32),
-            est=torch.zeros(B, Hkv, **f32),
-            aix=torch.zeros(B, Hkv, dtype=torch.uint8, device=dev),
-            idx=torch.zeros(B, NBC, dtype=torch.uint8, device=dev),
-            tlen=torch.zeros(B, dtype=torch.int32, device=dev),       # this step's lengths (ragged)
-            lens=torch.zeros(B, dtype=torch.int32, device=dev),       # all T, for batch_balance
-            part=torch.empty(E.plan_part_floats(B, Hq, Hkv, NBC), **f32),     # multi-workgroup plan
-            ticket=torch.zeros(B * Hkv, dtype=torch.int32, device=dev),      # one-launch plan (self-resetting)
-        )
+            part=torch.empty(E.plan_part_floats(B, Hq, Hkv, NBC), **f32))     # multi-workgroup plan
+        for h, f in enumerate(self.policy.flags(Hkv)):
+            if f:
+                self.state["flags"][h] = f
 
     def _grow(self, NBC):
         """src/kvskip_attn.py:435-442."""
