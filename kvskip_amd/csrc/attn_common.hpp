@@ -52,6 +52,8 @@
 // bounded to the head's rows, so rows past T read as zeros; their scores are masked to -inf.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -290,6 +292,27 @@ __device__ int global_lookup(const AttnP& p, int it, int& b, int& h, int& chunk,
   chunk = __builtin_amdgcn_readfirstlane(chunk);
   items = __builtin_amdgcn_readfirstlane(items);
   return C;
+}
+
+// Blocks per wavefront from which on a pass with V streams "long" (K taken direct, see KStage; the
+// rotation below short).
+constexpr int LONG_BLOCKS = 24;
+
+// Item of step k of a wavefront with nw > 0 items: k rotated by the workgroup's place in the grid (b, h and
+// the split alone, so passes that cut alike add alike). Without it every workgroup starts at the same
+// offset of its own range, and where the ranges lie at multiples of the memory's channel interleave apart
+// all of them read the same few channels at a time: B 1 at 64k in a buffer of 66048 tokens 74.0 -> 46.3 us
+// per op, of 65536 48.7 -> 45.4, B 2 at 64k (66048) 104.8 -> 85.7, single-pass V-skip at 64k 37.8 -> 26.3;
+// other sizes within 1%. Long streams drift apart by themselves, and spread further they lose locality:
+// rotated by up to 4 of their items B 8 at 64k takes 318 us, B 32 at 64k 1221 and at 60k 1113 (none: 328,
+// 1225, 1109; by up to all of them 312, 1242, 1110).
+__device__ __forceinline__ int item_rotation(const AttnP& p, int b, int h, int split, int nw) {
+  const int span = nw < LONG_BLOCKS ? nw : 4;
+  return nw > 0 ? __builtin_amdgcn_readfirstlane(((b * p.Hkv + h) * p.num_splits + split) % span) : 0;
+}
+__device__ __forceinline__ int rotated(int k, int rot, int nw) {
+  const int i = min(k, nw - 1) + rot;
+  return i >= nw ? i - nw : i;
 }
 
 // Byte range of one (b, head) of a K or V view: rows 0..T-1 of D bf16 each, row stride st.
@@ -599,11 +622,41 @@ struct MLay {
 // written and read in 8-byte pieces).
 __device__ __forceinline__ int mf_tok(int nt, int i, int j4) { return 16 * nt + 4 * j4 + i; }
 
-// Byte offset of this lane's K row within a 16-token tile (row lane % 16 of the A operand) and its
-// 16-byte chunk lane / 16.
+// K reaches the A operand's layout (16 rows x 64 bytes per k-step) in one of two ways.
+//   staged  loaded in whole rows (an instruction covers 512 / D rows of 2 D bytes) and passed through LDS, a
+//           16-token tile at a time. A tile is held as rows of D / 8 16-byte chunks, chunk c of row r at
+//           c ^ r (D 64: c ^ (r / 2)): a write fills whole rows and a read takes 16 different chunk places,
+//           so neither conflicts. Two tiles per wavefront.
+//   direct  loaded in the operand's layout: every instruction takes half lines of 16 rows.
+// Staged, a pass over K alone runs at 5.8 TB/s against 4.7 (B 8 at 32k 115.2 -> 94.0 us per op; D 64, 16 x 20k
+// 84.1 -> 70.1) and a short pass with V ends sooner (B 1 at 32k, 4 blocks per wavefront, 25.3 -> 24.0; 7 heads
+// 6 x 9k 25.7 -> 24.4; masked at 32k 15.1 -> 14.1). In a long pass with V, where both streams are in flight all
+// the time, the two ways of reading K and V at once move more: B 8 at 32k (32 blocks per wavefront) 159.3
+// staged, 155.0 direct; B 32 at 64k (256) 1249 and 1221; at 20 blocks per wavefront 101.7 and 102.6. So a
+// wavefront of a pass with V takes K direct from LONG_BLOCKS items on.
+template <int D>
+struct KStage {
+  static constexpr int TILE = 16 * 2 * D, TILES = 2, WAVE_BYTES = TILES * TILE, BYTES = NWAVE * WAVE_BYTES;
+};
+// Byte offset of this lane's row and chunk in a K load.
+template <int D, bool STAGED>
 __device__ __forceinline__ uint32_t mf_koff(int lane, int64_t k_st) {
-  return static_cast<uint32_t>((lane & 15) * k_st * 2 + 16 * (lane >> 4));
+  return STAGED ? static_cast<uint32_t>((lane / (D / 8)) * k_st * 2 + 16 * (lane % (D / 8)))
+                : static_cast<uint32_t>((lane & 15) * k_st * 2 + 16 * (lane >> 4));
 }
+// Byte offsets in a tile of this lane's part of load 0 (load kk: ^ 64 kk, + 1024 kk) and of its chunk of
+// k-step 0 (k-step kk: ^ 64 kk).
+template <int D>
+__device__ __forceinline__ uint32_t k_stage_w(int lane) {
+  const int r = lane / (D / 8), c = lane % (D / 8);
+  return static_cast<uint32_t>(r * 2 * D + 16 * (c ^ (D == 128 ? r : r >> 1)));
+}
+template <int D>
+__device__ __forceinline__ uint32_t k_stage_r(int lane) {
+  const int m = lane & 15, j4 = lane >> 4;
+  return static_cast<uint32_t>(m * 2 * D + 16 * (j4 ^ (D == 128 ? m : m >> 1)));
+}
+
 // V loads are 16 bytes (8 dims) per lane. D 128: a 16-lane group loads one row, load 4 nt + i the rows
 // mf_tok(nt, i, lane / 16), and column c holds dims 8 c .. + 7. D 64: a group loads two rows, load
 // 2 nt + i the tokens mf_tok(nt, 2 i, lane / 16) (lanes c < 8) and mf_tok(nt, 2 i + 1, ..) (c >= 8);
@@ -638,18 +691,18 @@ __device__ __forceinline__ float swap_sum(float v) {
   return __uint_as_float(t.x) + __uint_as_float(t.y);
 }
 
-// A operand (K) of one 64-token block: kr[nt][kk] = 16 bytes of this lane's row of tile nt at 16-byte
-// chunk 4 kk + lane/16. koffm = mf_koff.
-template <int D>
+// K of one 64-token block: kr[nt][kk] = this lane's row and chunk (mf_koff) of load kk of tile nt: staged, of
+// rows (512 / D) kk ..; direct, of chunks 4 kk ...
+template <int D, bool STAGED = true>
 __device__ __forceinline__ void load_k_block_mf(u32x4 (&kr)[4][MLay<D>::KS], rsrc_t rk, uint32_t koffm,
                                                 int64_t k_st, int t0) {
   const uint32_t rowb = static_cast<uint32_t>(k_st * 2);
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const uint32_t so = static_cast<uint32_t>(t0 + 16 * nt) * rowb;
+  for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-    for (int kk = 0; kk < MLay<D>::KS; ++kk) kr[nt][kk] = bload16<BUF_NT>(rk, koffm + 64 * kk, so);
-  }
+    for (int kk = 0; kk < MLay<D>::KS; ++kk)
+      kr[nt][kk] = STAGED ? bload16<BUF_NT>(rk, koffm, static_cast<uint32_t>(t0 + 16 * nt + (512 / D) * kk) * rowb)
+                          : bload16<BUF_NT>(rk, koffm + 64 * kk, static_cast<uint32_t>(t0 + 16 * nt) * rowb);
 }
 
 // V of one 64-token block. voffm = mf_voff.
@@ -690,18 +743,32 @@ __device__ __forceinline__ void load_q_mf(u32x4 (&qb)[MLay<D>::KS], const AttnP&
 }
 
 // Scores of one block in log2 units: s[nt][i] = head (lane % 16) % gpad, token t0 + mf_tok(nt, i,
-// lane / 16); tokens >= t_lim masked to -inf (only the block that t_lim cuts tests them).
-template <int D>
+// lane / 16); tokens >= t_lim masked to -inf (only the block that t_lim cuts tests them). sK: this
+// wavefront's KStage. A wavefront's LDS accesses complete in order, so a tile needs no wait between its
+// writes, its reads and the next tile's writes; the fences keep the compiler's order.
+template <int D, bool STAGED = true>
 __device__ __forceinline__ void qk_block_mf(float (&s)[4][4], const u32x4 (&kr)[4][MLay<D>::KS],
-                                            const u32x4 (&qb)[MLay<D>::KS], float scale_log2, int t0, int t_lim,
-                                            int lane) {
+                                            const u32x4 (&qb)[MLay<D>::KS], char* sK, float scale_log2, int t0,
+                                            int t_lim, int lane) {
+  constexpr int KS = MLay<D>::KS;
+  const uint32_t w0 = k_stage_w<D>(lane), r0 = k_stage_r<D>(lane);
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
+    char* tile = sK + (nt % KStage<D>::TILES) * KStage<D>::TILE;
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk)
+        *reinterpret_cast<u32x4*>(tile + 1024 * kk + (w0 ^ (64u * kk))) = kr[nt][kk];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
     f32x4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kk = 0; kk < MLay<D>::KS; ++kk)
-      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kr[nt][kk]),
-                                                  __builtin_bit_cast(bf16x8_t, qb[kk]), a, 0, 0, 0);
+    for (int kk = 0; kk < KS; ++kk) {
+      const u32x4 k = STAGED ? *reinterpret_cast<const u32x4*>(tile + (r0 ^ (64u * kk))) : kr[nt][kk];
+      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, k), __builtin_bit_cast(bf16x8_t, qb[kk]),
+                                                  a, 0, 0, 0);
+    }
+    if constexpr (STAGED) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[nt][i] = a[i] * scale_log2;
   }
@@ -864,10 +931,19 @@ __device__ __forceinline__ void pv_block_mf(PVAcc<D, G>& acc, const u32x4 (&vr)[
     }
 }
 
-// The MFMA engine's wavefront state into L (m, l: this lane's head's), then the merge.
+// LDS of an MFMA pass: the wavefronts' K tiles, then (after a barrier) the epilogue's states.
+template <int D, int G, bool LOAD_V>
+union MfLds {
+  char k[KStage<D>::BYTES];
+  MergeLds<D, G, LOAD_V ? PFrag<G>::NP : 0> merge;
+};
+
+// The MFMA engine's wavefront state into the epilogue's LDS (m, l: this lane's head's), then the merge.
 template <int D, int G, bool LOAD_V>
 __device__ __forceinline__ void finish_mf(const AttnP& p, float m, float l, const PVAcc<D, G>& acc, int b, int h,
-                                          int split, MergeLds<D, G, LOAD_V ? PFrag<G>::NP : 0>& L, bool plain) {
+                                          int split, MfLds<D, G, LOAD_V>& lds, bool plain) {
+  auto& L = lds.merge;
+  __syncthreads();  // every wavefront has left its K tiles
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int j4 = lane >> 4, c16 = lane & 15;
   if constexpr (LOAD_V) {

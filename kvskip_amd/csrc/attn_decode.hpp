@@ -306,8 +306,8 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
   static_assert(!PLANNED || MASKED, "a planned pass is masked");
   static_assert(!(PLANNED && RAG && PAGED), "a planned ragged pass reads a contiguous cache");
   static_assert(!PAGED || MF, "a paged cache is read by the MFMA engine");
-  constexpr int NP = LOAD_V ? (MF ? PFrag<G>::NP : 1) : 0;
-  __shared__ __attribute__((aligned(16))) MergeLds<D, G, NP> sL;
+  typedef std::conditional_t<MF, MfLds<D, G, LOAD_V>, MergeLds<D, G, LOAD_V ? 1 : 0>> Lds;
+  __shared__ __attribute__((aligned(16))) Lds sL;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
 
@@ -454,16 +454,17 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
   __shared__ int sBk[PAGED && MASKED ? MAX_NB : 1];
   if constexpr (PAGED)
     gather_pages(p, b, n, nbb, [&](int t) { return MASKED ? list(i0 + t) : i0 + t; }, sPg, MASKED ? sBk : nullptr);
-  // paged: item k of this wavefront (LDS slot wave + NWAVE k): its block and page
+  const int nw = n > wave ? (n - wave + NWAVE - 1) / NWAVE : 0;  // this wavefront's items
+  const int rot = item_rotation(p, b, h, split, nw);
+  // paged: item of step k of this wavefront (LDS slot wave + NWAVE item): its block and page
   auto paged_item = [&](int k, int& blk, int& pg) {
-    const int t = wave + NWAVE * k;
+    const int t = wave + NWAVE * rotated(k, rot, nw);
     pg = __builtin_amdgcn_readfirstlane(sPg[t]);
     if constexpr (MASKED)
       blk = __builtin_amdgcn_readfirstlane(sBk[t]);
     else
       blk = i0 + t;
   };
-  const int nw = n > wave ? (n - wave + NWAVE - 1) / NWAVE : 0;  // this wavefront's items
   int gap_prev = -1, gap_cur = 0;  // masked stats: the list entries around this lane's gap
   if constexpr (MASKED && STATS) {
     const int t = wave + NWAVE * lane;
@@ -477,19 +478,20 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
   const rsrc_t rv = make_rsrc(p.v + b * p.v_sb + h * p.v_sh, LOAD_V ? head_bytes(Tb, p.v_st, D) : 0);
   const int64_t hq0 = static_cast<int64_t>(b) * p.Hq + static_cast<int64_t>(h) * G;
 
-  // List entry of this wavefront's k-th item (k clamped to its items): a vector load whose value is
+  // List entry of this wavefront's step k (k clamped to its items): a vector load whose value is
   // used two items later, so that waiting for it never waits for the block loads issued after it.
-  auto entry_of = [&](int k) -> int { return MASKED ? list(i0 + wave + NWAVE * min(k, nw - 1)) : 0; };
-  // Block of the k-th item from its entry; out-of-range entries read block 0 and are masked.
+  auto entry_of = [&](int k) -> int { return MASKED ? list(i0 + wave + NWAVE * rotated(k, rot, nw)) : 0; };
+  // Block of step k from its entry; out-of-range entries read block 0 and are masked.
   auto block_of = [&](int e, int k) -> int {  // uniform over the wavefront
-    const int blk = __builtin_amdgcn_readfirstlane(MASKED ? e : i0 + wave + NWAVE * k);
+    const int blk = __builtin_amdgcn_readfirstlane(MASKED ? e : i0 + wave + NWAVE * rotated(k, rot, nw));
     return (blk >= 0 && blk < nbb) ? blk : -1;
   };
   if constexpr (MF) {
     // ---- MFMA engine: K(j + 1) is requested after the scores of block j, V(j + 1) after its P V.
     constexpr int KS = MLay<D>::KS;
     const int j4 = lane >> 4, c16 = lane & 15;
-    const uint32_t koffm = mf_koff(lane, p.k_st), voffm = mf_voff<D>(lane, p.v_st);
+    char* sK = sL.k + wave * KStage<D>::WAVE_BYTES;
+    const uint32_t koffm = mf_koff<D, true>(lane, p.k_st), voffm = mf_voff<D>(lane, p.v_st);
     // statistics and P of this (b, KV head) through buffer resources: one 32-bit offset per lane
     // (head c16: + c16 row bytes), the block in the scalar offset; out of range past the heads
     const uint32_t nb4 = 4u * static_cast<uint32_t>(p.nb), tp2 = 2u * static_cast<uint32_t>(p.t_pad);
@@ -497,7 +499,9 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     const rsrc_t rs_sum = make_rsrc(STATS ? p.blk_sum + hq0 * p.nb : nullptr, STATS ? G * nb4 : 0);
     const rsrc_t rs_p = make_rsrc(STATS && p.p_out != nullptr ? p.p_out + hq0 * p.t_pad : nullptr,
                                   STATS && p.p_out != nullptr ? G * tp2 : 0);
-    const uint32_t v_stat = c16 * nb4, v_p = c16 * tp2 + 8u * j4;
+    // offsets of a lane with nothing to store: past any range
+    constexpr uint32_t OOB = 0x80000000u;
+    const uint32_t v_stat = c16 < G && j4 == 0 ? c16 * nb4 : OOB, v_p = c16 < G ? c16 * tp2 + 8u * j4 : OOB;
     u32x4 qb[KS];
     load_q_mf<D, G>(qb, p, b, h, lane);
     float mr = NEG_INF, lr = 0.f;  // running (m, l) of this lane's head c16 % gpad
@@ -507,10 +511,11 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     // pf: its weights, alpha: the accumulators' rescale (this lane's head's). next_k: the K loads of the
     // block after it, into the registers its scores have just left. (Issued after the softmax: B 8 at 32k
     // 157.9 against 155.0 us per op; after P V: 159.7.)
-    auto process = [&](int blk, int lim, const u32x4 (&kr)[4][KS], PFrag<G>& pf, float& alpha, auto&& next_k) {
+    auto process = [&](auto staged, int blk, int lim, const u32x4 (&kr)[4][KS], PFrag<G>& pf, float& alpha,
+                       auto&& next_k) {
       const int t0 = blk >= 0 ? blk * BLK : 0;
       float s[4][4], e[4][4];
-      qk_block_mf<D>(s, kr, qb, p.scale_log2, t0, lim, lane);
+      qk_block_mf<D, decltype(staged)::value>(s, kr, qb, sK, p.scale_log2, t0, lim, lane);
       __builtin_amdgcn_sched_barrier(0);
       next_k();
       __builtin_amdgcn_sched_barrier(0);
@@ -523,19 +528,20 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
       lr = lr * alpha + st * cf;
       mr = m_new;
       if constexpr (STATS) {
-        if (blk >= 0 && c16 < G) {
-          if (j4 == 0) {
-            bstore_f32(mt * LN2, rs_max, v_stat, 4 * blk);
-            bstore_f32(st, rs_sum, v_stat, 4 * blk);
-          }
-          if (p.p_out != nullptr) {
+        // No branch around the stores (a lane or block without any stores out of range): a wait for loads
+        // on either side then counts them exactly (behind a branch, the wait for V(j) also covered the
+        // first K(j + 1) loads, requested just before it).
+        const uint32_t blk4 = 4u * static_cast<uint32_t>(max(blk, 0));
+        const uint32_t vs = blk >= 0 ? v_stat : OOB;
+        bstore_f32(mt * LN2, rs_max, vs, blk4);
+        bstore_f32(st, rs_sum, vs, blk4);
+        if (!LOAD_V || p.p_out != nullptr) {
+          const uint32_t vp = blk >= 0 ? v_p : OOB;
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) {
-              bstore_b64(u32x2{f2h(e[nt][0]) | static_cast<uint32_t>(f2h(e[nt][1])) << 16,
-                               f2h(e[nt][2]) | static_cast<uint32_t>(f2h(e[nt][3])) << 16},
-                         rs_p, v_p + 32 * nt, 2 * t0);
-            }
-          }
+          for (int nt = 0; nt < 4; ++nt)
+            bstore_b64(u32x2{f2h(e[nt][0]) | static_cast<uint32_t>(f2h(e[nt][1])) << 16,
+                             f2h(e[nt][2]) | static_cast<uint32_t>(f2h(e[nt][3])) << 16},
+                       rs_p, vp + 32 * nt, 2 * t0);
         }
       }
       if constexpr (LOAD_V) {
@@ -568,17 +574,16 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         load_k_block_mf<D>(ld, block_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, h, bld, gld, Tb, D), koffm, p.k_st,
                            max(bld, 0) * BLK);
         __builtin_amdgcn_sched_barrier(0);
-        if (k < nw) {
-          PFrag<G> pf;
-          float alpha;
-          process(bac, (bac >= 0 && gac >= 0) ? Tb : 0, ac, pf, alpha, [] {});
-        }
+        PFrag<G> pf;
+        float alpha;
+        process(std::true_type{}, bac, (bac >= 0 && gac >= 0) ? Tb : 0, ac, pf, alpha, [] {});
         __builtin_amdgcn_sched_barrier(0);
       };
-      for (int k = 0; k < nw; k += 2) {
+      for (int k = 0; k + 1 < nw; k += 2) {
         step(kb, b1, g1, ka, b0, g0, k);
         step(ka, b0, g0, kb, b1, g1, k + 1);
       }
+      if (nw % 2 != 0) step(kb, b1, g1, ka, b0, g0, nw - 1);
     } else if (nw > 0 && !LOAD_V) {
       // K only: two blocks in flight while one is scored (the V registers are free). Step k loads
       // item k + 1 and scores item k; past the last item the load reads beyond the head's buffer
@@ -594,71 +599,81 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         eb = ec;
         load_k_block_mf<D>(ld, rk, koffm, p.k_st, (k + 1 < nw ? max(bld, 0) : nbb) * BLK);
         __builtin_amdgcn_sched_barrier(0);
-        if (k < nw) {
-          PFrag<G> pf;
-          float alpha;
-          process(bac, bac >= 0 ? Tb : 0, ac, pf, alpha, [] {});
-        }
+        PFrag<G> pf;
+        float alpha;
+        process(std::true_type{}, bac, bac >= 0 ? Tb : 0, ac, pf, alpha, [] {});
         __builtin_amdgcn_sched_barrier(0);
       };
-      for (int k = 0; k < nw; k += 2) {
+      for (int k = 0; k + 1 < nw; k += 2) {
         step(kb, b1, ka, b0, k);
         step(ka, b0, kb, b1, k + 1);
       }
-    } else if (nw > 0 && PAGED) {
-      // each block's K / V resource spans its page's rows of this head that hold tokens (zeros
-      // beyond), an empty block's spans nothing; both are built before the block ahead is scored
-      // (built after it, the compiler spilled the freshly loaded K block)
-      u32x4 kr[4][KS];
-      u32x4 vr[MLay<D>::VN];
-      auto page_rsrc = [&](const uint16_t* pool, int64_t psb, int64_t sh, int64_t st, int blk, int pg) {
-        return block_rsrc(pool, psb, sh, st, h, blk, pg, Tb, D);
-      };
-      auto lim_of = [&](int blk, int pg) { return (blk >= 0 && pg >= 0) ? Tb : 0; };
-      int blk, pg;
-      paged_item(0, blk, pg);
-      load_k_block_mf<D>(kr, page_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, blk, pg), koffm, p.k_st, max(blk, 0) * BLK);
-      __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop: a wait for K is none for V
-      load_v_block_mf<D>(vr, page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk, pg), voffm, p.v_st, max(blk, 0) * BLK);
-      for (int k = 0; k < nw; ++k) {  // past the last item an empty block's loads (zeros, no memory access)
-        int blk_n = -1, pg_n = -1;
-        if (k + 1 < nw) paged_item(k + 1, blk_n, pg_n);
-        const rsrc_t rk_n = page_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, blk_n, pg_n);
-        const rsrc_t rv_n = page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk_n, pg_n);
-        PFrag<G> pf;
-        float alpha;
-        process(blk, lim_of(blk, pg), kr, pf, alpha,
-                [&] { load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, max(blk_n, 0) * BLK); });
-        accumulate(vr, pf, alpha);
-        __builtin_amdgcn_sched_barrier(0);
-        load_v_block_mf<D>(vr, rv_n, voffm, p.v_st, max(blk_n, 0) * BLK);
-        blk = blk_n;
-        pg = pg_n;
-      }
+      if (nw % 2 != 0) step(kb, b1, ka, b0, nw - 1);
     } else if (nw > 0) {
-      u32x4 kr[4][KS];
-      u32x4 vr[MLay<D>::VN];
-      int e_n = entry_of(1);
-      int blk = block_of(entry_of(0), 0);
-      load_k_block_mf<D>(kr, rk, koffm, p.k_st, max(blk, 0) * BLK);
-      __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop: a wait for K is none for V
-      load_v_block_mf<D>(vr, rv, voffm, p.v_st, max(blk, 0) * BLK);
-      // Every step issues the same loads; the last one's read beyond the head's buffer range (zeros, no
-      // memory access). (The last block peeled off the loop, or the loop left in its middle: the
-      // compiler spilled the first block's K and V on the way in, and waited for them there.)
-      for (int k = 0; k < nw; ++k) {
-        const int e_nn = entry_of(k + 2);
-        const int blk_n = block_of(e_n, min(k + 1, nw - 1));
-        const int t_n = (k + 1 < nw ? max(blk_n, 0) : nbb) * BLK;
-        e_n = e_nn;
-        PFrag<G> pf;
-        float alpha;
-        process(blk, blk >= 0 ? Tb : 0, kr, pf, alpha, [&] { load_k_block_mf<D>(kr, rk, koffm, p.k_st, t_n); });
-        accumulate(vr, pf, alpha);
-        __builtin_amdgcn_sched_barrier(0);
-        load_v_block_mf<D>(vr, rv, voffm, p.v_st, t_n);
-        blk = blk_n;
-      }
+      auto stream = [&](auto staged) {
+        constexpr bool ST = decltype(staged)::value;
+        const uint32_t koff = mf_koff<D, ST>(lane, p.k_st);
+        u32x4 kr[4][KS];
+        u32x4 vr[MLay<D>::VN];
+        if constexpr (PAGED) {
+          // each block's K / V resource spans its page's rows of this head that hold tokens (zeros
+          // beyond), an empty block's spans nothing; both are built before the block ahead is scored
+          // (built after it, the compiler spilled the freshly loaded K block)
+          auto page_rsrc = [&](const uint16_t* pool, int64_t psb, int64_t sh, int64_t st, int blk, int pg) {
+            return block_rsrc(pool, psb, sh, st, h, blk, pg, Tb, D);
+          };
+          auto lim_of = [&](int blk, int pg) { return (blk >= 0 && pg >= 0) ? Tb : 0; };
+          int blk, pg;
+          paged_item(0, blk, pg);
+          load_k_block_mf<D, ST>(kr, page_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, blk, pg), koff, p.k_st, max(blk, 0) * BLK);
+          __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop: a wait for K is none for V
+          load_v_block_mf<D>(vr, page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk, pg), voffm, p.v_st, max(blk, 0) * BLK);
+          for (int k = 0; k < nw; ++k) {  // past the last item an empty block's loads (zeros, no memory access)
+            int blk_n = -1, pg_n = -1;
+            if (k + 1 < nw) paged_item(k + 1, blk_n, pg_n);
+            const rsrc_t rk_n = page_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, blk_n, pg_n);
+            const rsrc_t rv_n = page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk_n, pg_n);
+            PFrag<G> pf;
+            float alpha;
+            process(staged, blk, lim_of(blk, pg), kr, pf, alpha,
+                    [&] { load_k_block_mf<D, ST>(kr, rk_n, koff, p.k_st, max(blk_n, 0) * BLK); });
+            accumulate(vr, pf, alpha);
+            __builtin_amdgcn_sched_barrier(0);
+            load_v_block_mf<D>(vr, rv_n, voffm, p.v_st, max(blk_n, 0) * BLK);
+            blk = blk_n;
+            pg = pg_n;
+          }
+        } else {
+          int e_n = entry_of(1);
+          int blk = block_of(entry_of(0), 0);
+          load_k_block_mf<D, ST>(kr, rk, koff, p.k_st, max(blk, 0) * BLK);
+          __builtin_amdgcn_sched_barrier(0);  // K before V, as in the loop: a wait for K is none for V
+          load_v_block_mf<D>(vr, rv, voffm, p.v_st, max(blk, 0) * BLK);
+          // Every step issues the same loads; the last one's read beyond the head's buffer range (zeros, no
+          // memory access). (The last block peeled off the loop, or the loop left in its middle: the
+          // compiler spilled the first block's K and V on the way in, and waited for them there.)
+          for (int k = 0; k < nw; ++k) {
+            const int e_nn = entry_of(k + 2);
+            const int blk_n = block_of(e_n, min(k + 1, nw - 1));
+            const int t_n = (k + 1 < nw ? max(blk_n, 0) : nbb) * BLK;
+            e_n = e_nn;
+            PFrag<G> pf;
+            float alpha;
+            process(staged, blk, blk >= 0 ? Tb : 0, kr, pf, alpha,
+                    [&] { load_k_block_mf<D, ST>(kr, rk, koff, p.k_st, t_n); });
+            accumulate(vr, pf, alpha);
+            __builtin_amdgcn_sched_barrier(0);
+            load_v_block_mf<D>(vr, rv, voffm, p.v_st, t_n);
+            blk = blk_n;
+          }
+        }
+      };
+      // (a planned pass takes K staged: its lists are short but for a refresh's, at most 16 lists' blocks
+      // over the whole GPU)
+      if (PLANNED || nw < LONG_BLOCKS)
+        stream(std::true_type{});
+      else
+        stream(std::false_type{});
     }
     finish_mf<D, G, LOAD_V>(p, mr, lr, acc, b, h, slot_base + split, sL, false);
   } else {

@@ -18,7 +18,8 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
   static_assert(!PAGED || MF, "a paged cache is read by the MFMA engine");
   constexpr int GP = gpad<G>();
   __shared__ int sPg[PAGED ? MAX_NB : 1];
-  __shared__ __attribute__((aligned(16))) MergeLds<D, G, MF ? PFrag<G>::NP : 1> sL;
+  typedef std::conditional_t<MF, MfLds<D, G, true>, MergeLds<D, G, 1>> Lds;
+  __shared__ __attribute__((aligned(16))) Lds sL;
   __shared__ float sLse0[G];
   __shared__ int sLoaded[NWAVE];
 
@@ -39,7 +40,8 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
     constexpr int KS = MLay<D>::KS;
     const int j4 = lane >> 4, c16 = lane & 15;
     const int hd = c16 % GP;  // this lane's head (none from G on)
-    const uint32_t koffm = mf_koff(lane, p.k_st), voffm = mf_voff<D>(lane, p.v_st);
+    char* sK = sL.k + wave * KStage<D>::WAVE_BYTES;
+    const uint32_t koffm = mf_koff<D, true>(lane, p.k_st), voffm = mf_voff<D>(lane, p.v_st);
     u32x4 qb[KS];
     load_q_mf<D, G>(qb, p, b, h, lane);
     u32x4 kr[4][KS];
@@ -65,7 +67,7 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
       }
       load_k_block_mf<D>(kr, krs(0, pg0), koffm, p.k_st, 0);
       float s[4][4], e[4][4];
-      qk_block_mf<D>(s, kr, qb, p.scale_log2, 0, lim_of(pg0), lane);
+      qk_block_mf<D>(s, kr, qb, sK, p.scale_log2, 0, lim_of(pg0), lane);
       const float mt = block_max_mf(s);  // an empty block 0 (paged): -inf, every block kept
       const float sum = block_exp_mf(e, s, mt);
       if (j4 == 0 && c16 < G) sLse0[c16] = (mt == NEG_INF ? 0.f : mt) + flog2(sum);
@@ -75,24 +77,26 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
       lse0 = sLse0[min(hd, G - 1)];
     }
     float mr = NEG_INF, lr = 0.f;
-    // Item k of this wavefront is block i0 + wave + 4 k: K of the next item is requested right after the
+    // K of the next item is requested right after the
     // scores (past the last item beyond the head's range: zeros, no memory access), V only if the group
     // keeps the block. Measured (op, us; B 8 at 32k nothing kept / 64k peaked): the P V by FMAs and K
     // requested after the vote 98.3 / 44.6; P V on MFMA 93.9 / 42.2; K requested after the scores 91.8 /
     // 42.2. V requested always (out of range where not kept) and used a step later: 113.0.
-    int pg = nw > 0 ? page_at(wave) : -1;
-    if (nw > 0) load_k_block_mf<D>(kr, krs(i0 + wave, pg), koffm, p.k_st, (i0 + wave) * BLK);
+    const int rot = item_rotation(p, b, h, split, nw);
+    auto slot_of = [&](int k) { return wave + NWAVE * rotated(k, rot, nw); };  // of step k: block i0 + slot
+    int pg = nw > 0 ? page_at(slot_of(0)) : -1;
+    if (nw > 0) load_k_block_mf<D>(kr, krs(i0 + slot_of(0), pg), koffm, p.k_st, (i0 + slot_of(0)) * BLK);
     for (int k = 0; k < nw; ++k) {
-      const int blk = i0 + wave + NWAVE * k;
+      const int blk = i0 + slot_of(k);
       const bool more = k + 1 < nw;
       // this block's V and the next block's K resources, built before the scores
-      const int pg_n = more ? page_at(wave + NWAVE * (k + 1)) : -1;
-      const rsrc_t rv_c = vrs(blk, pg), rk_n = krs(blk + NWAVE, pg_n);
+      const int blk_n = i0 + slot_of(k + 1), pg_n = more ? page_at(slot_of(k + 1)) : -1;
+      const rsrc_t rv_c = vrs(blk, pg), rk_n = krs(blk_n, pg_n);
       float s[4][4], e[4][4];
-      qk_block_mf<D>(s, kr, qb, p.scale_log2, blk * BLK, lim_of(pg), lane);
+      qk_block_mf<D>(s, kr, qb, sK, p.scale_log2, blk * BLK, lim_of(pg), lane);
       pg = pg_n;
       __builtin_amdgcn_sched_barrier(0);
-      load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, (PAGED || more ? blk + NWAVE : nb) * BLK);
+      load_k_block_mf<D>(kr, rk_n, koffm, p.k_st, (PAGED || more ? blk_n : nb) * BLK);
       __builtin_amdgcn_sched_barrier(0);
       const float mt = block_max_mf(s);
       const float mtu = mt == NEG_INF ? 0.f : mt;
@@ -247,7 +251,7 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
                                         ScaleAt scale_at) {
   __shared__ int sPg[PAGED ? MAX_NB : 1];
   __shared__ int sBk[PAGED ? MAX_NB : 1];
-  __shared__ __attribute__((aligned(16))) MergeLds<D, G, PFrag<G>::NP> sL;
+  __shared__ __attribute__((aligned(16))) MfLds<D, G, true> sL;
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int per = (n_items + p.num_splits - 1) / p.num_splits;
