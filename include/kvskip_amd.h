@@ -107,6 +107,14 @@ typedef struct kvskip_attn_args {
    * num_splits)), so a KV head whose lists hold more entries gets more workgroups (needs
    * B * Hkv <= 512). The merge (kvskip_merge_splits) must be given the value its pass had. */
   int32_t list_partition;
+
+  /* Per-block key sums beside the pass (not in the reference; kvskip_decode and kvskip_decode_splits, dense
+   * with statistics over a contiguous ragged batch: seq_lens, no block_idx, no block_table): optional fp32
+   * [B, Hkv, sums_cap, D], sums_cap >= ceil(T / 64); each block of a sequence gets the sum of its rows, as
+   * kvskip_block_sums writes it, from the K that the pass reads anyway. Blocks past a sequence's end are
+   * not written. */
+  float* key_sums;
+  int32_t sums_cap;
 } kvskip_attn_args;
 
 /* Split-K decode attention: dense (block_idx NULL) or over block lists, with optional per-block

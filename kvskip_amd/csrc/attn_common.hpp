@@ -705,6 +705,32 @@ __device__ __forceinline__ void load_k_block_mf(u32x4 (&kr)[4][MLay<D>::KS], rsr
                           : bload16<BUF_NT>(rk, koffm + 64 * kk, static_cast<uint32_t>(t0 + 16 * nt) * rowb);
 }
 
+// Sum over the rows of a block loaded staged (load_k_block_mf), for this lane's 8 dims 8 (lane % (D / 8)): pairs
+// of rows by v_perm, added by v_dot2_f32_bf16 against ones (exact products, fp32 sums), then over the lanes that
+// hold the chunk's other rows. About 210 instructions per block beside a stream that waits for memory.
+// Measured (first step of a layer, us, pass + sums apart -> together): 32 x 40k, 32 / 8 heads, 776 + 491 -> 914;
+// 16 ragged sequences to 64k, 28 / 4 heads, 134 + 102 -> 155.
+template <int D>
+__device__ __forceinline__ void block_key_sums(const u32x4 (&kr)[4][MLay<D>::KS], float (&sum)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+    for (int kk = 0; kk < MLay<D>::KS; kk += 2)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t a = kr[nt][kk][d], c = kr[nt][kk + 1][d];
+        sum[2 * d] = dot2(__builtin_amdgcn_perm(c, a, 0x05040100u), 0x3f803f80u, sum[2 * d]);
+        sum[2 * d + 1] = dot2(__builtin_amdgcn_perm(c, a, 0x07060302u), 0x3f803f80u, sum[2 * d + 1]);
+      }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    if constexpr (D == 64) sum[e] += dpp<DPP_ROR8>(sum[e]);
+    sum[e] = swap_sum(sum[e]);
+  }
+}
+
 // V of one 64-token block. voffm = mf_voff.
 template <int D>
 __device__ __forceinline__ void load_v_block_mf(u32x4 (&vr)[MLay<D>::VN], rsrc_t rv, uint32_t voffm, int64_t v_st,

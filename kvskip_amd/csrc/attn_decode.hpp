@@ -301,11 +301,13 @@ __device__ bool planned_ragged(const AttnP& p, const kvskip_plan_args& pa, int h
 // comes from device memory; the grid is still num_splits x Hkv x B. With pa->pass_budget > 0 the
 // prologue is planned_balanced's instead (grid pass_budget + B Hkv, num_splits partial slots).
 template <int D, int G, bool MASKED, bool STATS, bool LOAD_V, bool MF, bool RAG, bool PLANNED = false,
-          bool PAGED = false>
-__device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvskip_plan_args* pa = nullptr) {
+          bool PAGED = false, bool SUMS = false>
+__device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvskip_plan_args* pa = nullptr,
+                                            float* sums = nullptr, int sums_cap = 0) {
   static_assert(!PLANNED || MASKED, "a planned pass is masked");
   static_assert(!(PLANNED && RAG && PAGED), "a planned ragged pass reads a contiguous cache");
   static_assert(!PAGED || MF, "a paged cache is read by the MFMA engine");
+  static_assert(!SUMS || (MF && RAG && STATS && LOAD_V && !MASKED && !PAGED), "key sums: a dense ragged pass with statistics");
   typedef std::conditional_t<MF, MfLds<D, G, LOAD_V>, MergeLds<D, G, LOAD_V ? 1 : 0>> Lds;
   __shared__ __attribute__((aligned(16))) Lds sL;
 
@@ -557,6 +559,16 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
       rescale_acc<D, G>(acc, alpha, lane);
       pv_block_mf<D, G>(acc, vr, pf, lane);
     };
+    // key sums (kvskip_attn_args.key_sums) of block blk from its K, loaded staged
+    const rsrc_t rs_ks = make_rsrc(SUMS ? sums + (static_cast<int64_t>(b) * p.Hkv + h) * sums_cap * D : nullptr,
+                                   SUMS ? static_cast<uint32_t>(sums_cap) * D * 4 : 0);
+    auto key_sums = [&](int blk, const u32x4 (&kr)[4][KS]) {
+      float ks[8];
+      block_key_sums<D>(kr, ks);
+      const uint32_t off = lane < D / 8 ? 32u * lane : OOB, so = static_cast<uint32_t>(max(blk, 0)) * D * 4;
+      bstore16_f32(ks[0], ks[1], ks[2], ks[3], rs_ks, off, so);
+      bstore16_f32(ks[4], ks[5], ks[6], ks[7], rs_ks, off + 16, so);
+    };
     if (nw > 0 && !LOAD_V && PAGED) {
       // K only over a paged cache: two blocks in flight as below, each through its page's resource
       u32x4 ka[4][KS], kb[4][KS];
@@ -660,7 +672,10 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
             PFrag<G> pf;
             float alpha;
             process(staged, blk, blk >= 0 ? Tb : 0, kr, pf, alpha,
-                    [&] { load_k_block_mf<D, ST>(kr, rk, koff, p.k_st, t_n); });
+                    [&] {
+                      if constexpr (SUMS) key_sums(blk, kr);
+                      load_k_block_mf<D, ST>(kr, rk, koff, p.k_st, t_n);
+                    });
             accumulate(vr, pf, alpha);
             __builtin_amdgcn_sched_barrier(0);
             load_v_block_mf<D>(vr, rv, voffm, p.v_st, t_n);
@@ -669,8 +684,8 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         }
       };
       // (a planned pass takes K staged: its lists are short but for a refresh's, at most 16 lists' blocks
-      // over the whole GPU)
-      if (PLANNED || nw < LONG_BLOCKS)
+      // over the whole GPU; key sums add up whole rows)
+      if (PLANNED || SUMS || nw < LONG_BLOCKS)
         stream(std::true_type{});
       else
         stream(std::false_type{});

@@ -170,6 +170,12 @@ static int check_decode(const kvskip_attn_args* a, int stats, int load_v, int ph
     if (a->B > kvs::MAX_RAGGED_B) return fail(KVSKIP_E_UNSUPPORTED, "seq_lens: B <= %d", kvs::MAX_RAGGED_B);
     if (a->p_out != nullptr) return fail(KVSKIP_E_UNSUPPORTED, "seq_lens: no fp16 P output");
   }
+  if (a->key_sums != nullptr && (phase & 1)) {
+    if (masked || !stats || !load_v || a->p_out != nullptr || a->seq_lens == nullptr || a->block_table != nullptr)
+      return fail(KVSKIP_E_UNSUPPORTED, "key_sums: a dense pass with statistics over a contiguous ragged batch");
+    if (a->sums_cap < p->nb || !aligned16(a->key_sums))
+      return fail(KVSKIP_E_INVALID, "key_sums: 16-byte aligned [B, Hkv, sums_cap >= ceil(T / 64), D]");
+  }
   if (a->list_partition != 0) {
     if (a->list_partition != 1) return fail(KVSKIP_E_INVALID, "list_partition in {0, 1}");
     if (!masked || a->seq_lens == nullptr)
@@ -190,6 +196,9 @@ static int decode_phases(const kvskip_attn_args* a, int stats, int load_v, int p
   const int rc = check_decode(a, stats, load_v, phase, &p);
   if (rc != KVSKIP_OK) return rc;
   const int G = a->Hq / a->Hkv;
+  if (a->key_sums != nullptr && (phase & 1))
+    return launched(kvs::launch_decode_sums(p, a->D, G, a->key_sums, a->sums_cap, phase, static_cast<hipStream_t>(stream)),
+                    "kvskip_decode");
   return launched(kvs::launch_decode(p, a->D, G, a->block_idx != nullptr, stats != 0, load_v != 0, phase,
                                      static_cast<hipStream_t>(stream)),
                   "kvskip_decode");

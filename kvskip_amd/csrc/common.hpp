@@ -173,6 +173,11 @@ __device__ __forceinline__ void bstore_u16(uint16_t v, rsrc_t r, uint32_t voff, 
 __device__ __forceinline__ void bstore_b64(u32x2 v, rsrc_t r, uint32_t voff, uint32_t soff) {
   __builtin_amdgcn_raw_buffer_store_b64(v, r, static_cast<int>(voff), static_cast<int>(soff), 0);
 }
+__device__ __forceinline__ void bstore16_f32(float a, float b, float c, float d, rsrc_t r, uint32_t voff,
+                                             uint32_t soff) {
+  __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), __float_as_uint(d)},
+                                         r, static_cast<int>(voff), static_cast<int>(soff), 0);
+}
 
 // Online log-sum-exp accumulator in natural units (planner): (m, s) with s = sum exp(x - m).
 __device__ __forceinline__ void lse_push(float& m, float& s, float x) {

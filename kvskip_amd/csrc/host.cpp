@@ -334,7 +334,7 @@ void pass_bufs(Outs& o, PyObject* bufs, bool stats, int64_t S, const Dims& d, bo
 }
 
 // decode_into(q, k, v, scale, bufs, block_idx, block_cnt, stats, num_splits, seq_lens, phase, block_table, T,
-//             list_partition)
+//             list_partition, key_sums)
 PyObject* decode_into(PyObject* const* a) {
   const at::Tensor &q = tensor(a[0], "q"), &k = tensor(a[1], "k"), &v = tensor(a[2], "v");
   check_q(q);
@@ -354,6 +354,12 @@ PyObject* decode_into(PyObject* const* a) {
   kvskip_attn_args args;
   set_decode(args, q, k, v, real(a[3]), opt_tensor(a[5], "block_idx"), opt_tensor(a[6], "block_cnt"), S, o,
              opt_tensor(a[9], "seq_lens"), bt, a[12], int32(a[13]));
+  if (const at::Tensor* t = opt_tensor(a[14], "key_sums")) {
+    check_f32(*t, "key_sums");
+    require(t->dim() == 4 && t->size(0) == d.B && t->size(1) == d.Hkv && t->size(2) >= d.nb && t->size(3) == d.D,
+            "key_sums: [B, Hkv, >= ceil(T / 64), D]");
+    args.key_sums = static_cast<float*>(t->data_ptr()), args.sums_cap = static_cast<int32_t>(t->size(2));
+  }
   auto* fn = phase == 3 ? api.decode : phase == 1 ? api.decode_splits : phase == 2 ? api.merge_splits : nullptr;
   require(fn != nullptr, "phase in {1, 2, 3}");
   launch(q.device(), [&](void* s) { return fn(&args, stats, 1, s); });
@@ -857,7 +863,7 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 #define KVS_FN(f, n) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call<f, n>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bind)), METH_FASTCALL, nullptr},
-    KVS_FN(decode, 17), KVS_FN(decode_into, 14), KVS_FN(splits_planned, 14), KVS_FN(splits_update, 13),
+    KVS_FN(decode, 17), KVS_FN(decode_into, 15), KVS_FN(splits_planned, 14), KVS_FN(splits_update, 13),
     KVS_FN(attn_block, 20), KVS_FN(vskip1, 13), KVS_FN(select, 10), KVS_FN(pv, 9), KVS_FN(pv_select, 13),
     KVS_FN(plan_block, 33), KVS_FN(update_block, 24), KVS_FN(plan, 2), KVS_FN(merge_update, 3), KVS_FN(plan_scores, 2),
     KVS_FN(update, 2), KVS_FN(num_splits, 5), KVS_FN(zeroed, 2),

@@ -105,15 +105,17 @@ def decode(q, k, v, scale, block_idx=None, block_cnt=None, stats=False, load_v=T
 
 
 def decode_into(q, k, v, scale, bufs: dict, block_idx=None, block_cnt=None, stats=False, num_splits=1,
-                seq_lens=None, phase=3, block_table=None, T=None, list_partition=0):
+                seq_lens=None, phase=3, block_table=None, T=None, list_partition=0, key_sums=None):
     """decode() into caller-owned buffers, allocating nothing (not in the reference): bufs holds
     out bf16, lse fp32 and, as needed, blk_max / blk_sum fp32 (>= B*Hq*nb elements, written as
     [B, Hq, nb], -inf / 0 where a list skips a block) and part_acc / part_ml fp32
     (>= B*Hq*num_splits*D / *2 elements). The fused planner loop runs its passes this way.
     phase: 3 = the whole op, 1 = the split pass only (its merge left to merge_splits / merge_update),
-    2 = that merge alone (given the pass's list_partition). block_table, T: a paged cache."""
+    2 = that merge alone (given the pass's list_partition). block_table, T: a paged cache.
+    key_sums: fp32 [B, Hkv, NBC, D]; a dense pass with stats and seq_lens also writes block_sums' sums of the
+    sequences' blocks there (kvskip_attn_args.key_sums; blocks past a sequence's end are left alone)."""
     _host().decode_into(q, k, v, scale, bufs, block_idx, block_cnt, stats, num_splits, seq_lens, phase, block_table, T,
-                        list_partition)
+                        list_partition, key_sums)
 
 
 class DecodeOp:

@@ -32,6 +32,10 @@ BALANCE_MAX_LISTS = 16           # (b, KV head) lists a balanced planned pass de
 RAGGED_DECIDE_MAX_B = 16         # sequences of a ragged batch whose lists a planned pass decides per KV head
 GLOBAL_PARTITION_MAX_LISTS = 512  # B * Hkv bound of kvskip_attn_args.list_partition = 1
 GLOBAL_PARTITION_MAX_B = 64        # sequences up to which the planner cuts all heads' lists together
+# Blocks of K (B * Hkv * nb; 256 MiB of 128-dim keys) from which on a batch's first step sums the keys in its dense
+# pass instead of a pass of their own: below, K is still in the cache for the second reading and the update rides
+# on the next layer's pass instead of beside the merge
+SUMS_IN_PASS_BLOCKS = 16384
 POST_MAX_SLOTS = 64              # first-pass partial slots the refresh mode's decision reads (lse_slots)
 KINDS = {"logit": 0, "add": 1, "peak": 2}
 
@@ -206,14 +210,15 @@ class FusedPlanner:
         self.state["part"] = torch.empty(E.plan_part_floats(B, Hq, Hkv, NBC), dtype=torch.float32, device=idx.device)
         self.NBC = NBC
 
-    def _attend(self, q, k, v, scale, nb, seq_lens=None):
-        pg = self._pg
-        """Split pass (masked + statistics) over the plan's lists into the planner's buffers.
+    def _attend(self, q, k, v, scale, nb, seq_lens=None, key_sums=None):
+        """Split pass (masked + statistics) over the plan's lists into the planner's buffers; with
+        key_sums over every block, the blocks' key sums written there.
         Returns out [B, Hq, D] (valid until the next step; written by _finish when the pass is
         split) and the [B, Hq, nb] statistics views."""
+        pg = self._pg
         B, Hq, D = q.shape
         Hkv = k.shape[1]
-        carried = self.carrier.take(self, Hq // Hkv) if self.carrier is not None else None
+        carried = self.carrier.take(self, Hq // Hkv) if self.carrier is not None and key_sums is None else None
         # one sequence (its length in device memory) is split as an unragged batch
         S = (K.num_splits_for(B * Hkv, nb) if seq_lens is None or B == 1
              else K.ragged_splits(B, Hkv, nb, G=Hq // Hkv, carry=carried is not None))
@@ -246,11 +251,13 @@ class FusedPlanner:
                                  part_ml=torch.empty(B * Hq * S_buf * 2, **f32))
         s = self.state
         self._S = S
-        self._lp = lp = int(self._pargs is None and self.global_partition and seq_lens is not None
+        self._lp = lp = int(self._pargs is None and key_sums is None and self.global_partition and seq_lens is not None
                             and 1 < B <= GLOBAL_PARTITION_MAX_B and B * Hkv <= GLOBAL_PARTITION_MAX_LISTS)
         if self._pargs is not None:
             self._pargs.pass_budget = budget
             E.decode_splits_planned(q, k, v, scale, b, self._pargs, S, carried, seq_lens, **pg)
+        elif key_sums is not None:
+            E.decode_into(q, k, v, scale, b, stats=True, num_splits=S, seq_lens=seq_lens, phase=1, key_sums=key_sums)
         elif carried is not None:
             E.decode_splits_update(q, k, v, scale, b, s["block_idx"], s["block_cnt"], S, carried, seq_lens,
                                    list_partition=lp, **pg)
@@ -260,11 +267,15 @@ class FusedPlanner:
         n = B * Hq * nb
         return b["out"], b["blk_max"][:n].view(B, Hq, nb), b["blk_sum"][:n].view(B, Hq, nb)
 
-    def _finish(self, q, k, v, scale, seq_lens, update_args, update_kwargs):
+    def _finish(self, q, k, v, scale, seq_lens, update_args, update_kwargs, dense=False):
         """The pass's split merge and the planner update: one launch (kvskip_merge_update) when
         the pass was split, else the update alone; with a carrier, the merge alone and the update
-        left to the next layer's pass."""
+        left to the next layer's pass. dense: a pass over every block, which carried no update and leaves
+        its own to no other."""
         s = self.state
+        if dense:
+            E.merge_update(q, k, v, scale, self.bufs, self._S, update_args, update_kwargs, seq_lens=seq_lens)
+            return
         if self.carrier is not None:
             if self._S > 1:
                 E.decode_into(q, k, v, scale, self.bufs, s["block_idx"], s["block_cnt"], stats=True,
@@ -279,7 +290,7 @@ class FusedPlanner:
         else:
             E.update(*update_args, **update_kwargs)
 
-    def _plan(self, q, plan_args, plan_kwargs, seq_lens):
+    def _plan(self, q, plan_args, plan_kwargs, seq_lens, in_pass=True):
         """plan (scores + decision), or, with decide_in_pass, its scores pass alone: the decision then
         runs in the masked pass (kvskip_decode_splits_planned) and the update advances the age. A
         ragged batch decides in the pass as ragged_in_pass says (up to RAGGED_DECIDE_MAX_B sequences
@@ -287,7 +298,7 @@ class FusedPlanner:
         decides."""
         B = q.shape[0]
         rag = bool(self.ragged_in_pass)
-        if self.decide_in_pass and (seq_lens is None or B == 1
+        if in_pass and self.decide_in_pass and (seq_lens is None or B == 1
                                     or (rag and B <= RAGGED_DECIDE_MAX_B and not self._pg)):
             self._pargs = E.plan_struct(*plan_args, **plan_kwargs)
             E.plan_scores(self._pargs, q.device)
@@ -353,18 +364,28 @@ class FusedPlanner:
         self._alloc(q, k, nb + MARGIN)
         s = self.state
         seq_lens = self._batch_lens(B, Hkv, T, seq_lens, block_table)
-        E.block_sums(k, self.NBC, out=s["csum"], seq_lens=seq_lens, **self._pg)
         every = torch.ones(Hkv, dtype=torch.int32, device=q.device)      # refresh all, no index heads
         pol = self.policy
+        sums_in_pass = seq_lens is not None and block_table is None and B > 1 and B * Hkv * nb >= SUMS_IN_PASS_BLOCKS
+        if sums_in_pass:
+            self._pargs = None
+            # dense pass first, the key sums from the K that it reads; then the plan (every head
+            # refreshes, whatever its estimate), then the merge and the update
+            s["csum"][:, :, nb if seq_lens is s["lens"] else 0:].zero_()
+            out, bmax, bsum = self._attend(q, k, v, scale, nb, seq_lens, key_sums=s["csum"])
+        else:
+            E.block_sums(k, self.NBC, out=s["csum"], seq_lens=seq_lens, **self._pg)
         self._plan(q, (q, k, s["csum"], s["lse_ref"], s["cs_ref"], s["keep"], s["lse_att"], s["age"], every,
                        s["cs_now"], s["trig"], s["block_idx"], s["block_cnt"], float(scale), float(pol.delta),
                        int(pol.max_age), int(pol.local), False),
-                   dict(part=s["part"], seq_lens=seq_lens, seq_lens_out=self._tlen(seq_lens), **self._pg), seq_lens)
-        out, bmax, bsum = self._attend(q, k, v, scale, nb, seq_lens)
+                   dict(part=s["part"], seq_lens=seq_lens, seq_lens_out=self._tlen(seq_lens), **self._pg), seq_lens,
+                   in_pass=not sums_in_pass)
+        if not sums_in_pass:
+            out, bmax, bsum = self._attend(q, k, v, scale, nb, seq_lens)
         self._finish(q, k, v, scale, seq_lens,
                      (bmax, bsum, s["trig"], s["cs_now"], s["keep"], s["lse_ref"], s["cs_ref"], s["lse_att"], T,
                       float(pol.level), int(pol.local), every),
-                     dict(list_stats=True, seq_lens=self._tlen(seq_lens), **self._age()))
+                     dict(list_stats=True, seq_lens=self._tlen(seq_lens), **self._age()), dense=sums_in_pass)
         self.t, self.T = 0, T
         self.ragged = seq_lens is not None and seq_lens is not s["lens"]
         if self.count:
