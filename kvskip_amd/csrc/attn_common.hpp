@@ -303,9 +303,11 @@ constexpr int LONG_BLOCKS = 24;
 // offset of its own range, and where the ranges lie at multiples of the memory's channel interleave apart
 // all of them read the same few channels at a time: B 1 at 64k in a buffer of 66048 tokens 74.0 -> 46.3 us
 // per op, of 65536 48.7 -> 45.4, B 2 at 64k (66048) 104.8 -> 85.7, single-pass V-skip at 64k 37.8 -> 26.3;
-// other sizes within 1%. Long streams drift apart by themselves, and spread further they lose locality:
+// other short ones within 1%. Long streams drift apart by themselves, and spread further they lose locality:
 // rotated by up to 4 of their items B 8 at 64k takes 318 us, B 32 at 64k 1221 and at 60k 1113 (none: 328,
-// 1225, 1109; by up to all of them 312, 1242, 1110).
+// 1225, 1109; by up to all of them 312, 1242, 1110). Where a head is one split the choice
+// depends on the stride: B 32 at 65536 1246 - 1269 us (none 1270 - 1302), at 48000 of 49152 945 - 951 (962 -
+// 976), at 65552 of 65568 1276 - 1301 (1233 - 1265).
 __device__ __forceinline__ int item_rotation(const AttnP& p, int b, int h, int split, int nw) {
   const int span = nw < LONG_BLOCKS ? nw : 4;
   return nw > 0 ? __builtin_amdgcn_readfirstlane(((b * p.Hkv + h) * p.num_splits + split) % span) : 0;
