@@ -33,8 +33,8 @@
 //         lane / 16). V is read with 8 (D 64: 4) dims of a row per lane; two rows' halves are paired by
 //         v_perm into B operands whose column c is dim 8 c + j. Weights stay fp32: a weight is the exact
 //         sum of three bf16 parts (hi, mid, lo: 8 + 8 + 8 bits), and since the group's G <= 8 heads leave
-//         rows free, the 16 rows are the parts of the heads (4 heads x 3 parts, or 8 heads x hi, mid and
-//         a second product for lo): three parts for the price of one product. The products are exact and
+//         rows free, the 16 rows are the parts of the heads (4 heads x 3 parts in one product, or 8 heads
+//         x 2 in two: hi / 2 and mid, hi / 2 and lo). The products are exact and
 //         summed in fp32, as the VALU engine's.
 //         What it replaced: P through LDS and G x 128 FMAs plus 128 conversions per lane and block
 //         (D 128), which at G 7 took longer than the block's loads (figures at PFrag below).
@@ -836,10 +836,12 @@ __device__ __forceinline__ float block_exp_mf(float (&e)[4][4], const float (&s)
 // rounded from, where the compiler contracts).
 //   4-head groups   one product, parts (hi, mid, lo, 0): the weight's top 8 significant bits, the next 8
 //                   and the rest, each by truncation.
-//   8-head groups   two products into the same accumulators, parts (hi, mid) then (lo / 2, lo / 2), cut one
-//                   bit lower so that no part of a weight > 0 is 0 (see sat_dec).
-// An infinite V entry meets a part that is 0 only where the weight is 0, or (4-head groups) in rows that
-// merged_acc leaves out then, so it gives the infinity that an fp32 product gives and no NaN.
+//   8-head groups   two products into the same accumulators, parts (hi / 2, mid) then (hi / 2, lo).
+// An infinite V entry times a part that is 0 is NaN. Part 0 is hi alone, and merged_acc takes part 0 alone
+// where it is infinite, so the infinity of an fp32 product comes out for every weight whose hi (8-head
+// groups: hi / 2) is a bf16 other than 0: any |weight| >= 2^-125, whether or not the unit keeps bf16
+// denormals (weights below 2^-126 only arise as products of a token's and its block's factors). The lo / 2
+// in both parts that this replaced was 0 from about 2^-109 on.
 // Measured against P through LDS and P V as fp32 FMAs (G x 128 per lane and block at D 128, and 128
 // conversions; op, us, graph-replayed): B 1 at 32k 26.6 -> 25.9 dense, 16.3 -> 14.9 masked with statistics
 // (35% listed); 7 heads, B 6 at 9k, 27.6 -> 24.7; 8 heads, B 4 at 16k, 48.6 -> 45.8; D 64 at 4k 8.7 -> 7.6;
@@ -856,9 +858,6 @@ __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
   return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 constexpr uint32_t BF_HI = 0xffff0000u;
-// The largest float below a (a > 0; 0 stays 0): truncated to bf16 it is below a by at most 2 ulps of bf16
-// and above 0, and a less it is exact and above 0.
-__device__ __forceinline__ uint32_t sat_dec(uint32_t a) { return __builtin_elementwise_sub_sat(a, 1u); }
 
 // The lane's column gives weight 0 where this is false (the unused fourth part of 4-head groups).
 template <int G>
@@ -871,6 +870,7 @@ __device__ __forceinline__ PFrag<G> make_frag(const float (&w)[4][4], int lane) 
   PFrag<G> f;
   const int part = (lane & 15) / gpad<G>();
   const uint32_t m1 = part >= 1 ? BF_HI : 0u, m2 = part >= 2 ? BF_HI : 0u;
+  const float half = part == 0 ? 0.5f : 1.f;  // 8-head groups
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -879,14 +879,11 @@ __device__ __forceinline__ PFrag<G> make_frag(const float (&w)[4][4], int lane) 
 #pragma unroll
       for (int o = 0; o < 2; ++o) {
         const float a = w[2 * s + u / 2][2 * (u % 2) + o];
+        const float r = a - __uint_as_float(__float_as_uint(a) & m1);  // part 0: the weight itself
         if constexpr (gpad<G>() == 8) {
-          const uint32_t h = sat_dec(__float_as_uint(a));
-          const float r = a - __uint_as_float(h & BF_HI);
-          const uint32_t m = sat_dec(__float_as_uint(r));
-          v[o] = part != 0 ? m : h;
-          lo[o] = __float_as_uint(0.5f * (r - __uint_as_float(m & BF_HI)));
+          v[o] = __float_as_uint(half * r);
+          lo[o] = __float_as_uint(half * r - __uint_as_float(v[o] & m1));
         } else {
-          const float r = a - __uint_as_float(__float_as_uint(a) & m1);
           v[o] = __float_as_uint(r - __uint_as_float(__float_as_uint(r) & m2));
         }
       }
