@@ -66,8 +66,9 @@ typedef struct kvskip_attn_args {
   float* blk_max;
   float* blk_sum;
 
-  /* two-pass V-skip: pass 1 writes P = exp(s - blk_max) as fp16 [B, Hq, nb*64];
-   * pass 2 reads it back with blk_scale [B, Hkv, nb, G] */
+  /* two-pass V-skip: pass 1 writes P = exp(s - blk_max) as fp16 [B, Hq, nb*64] (p_out at any fp16
+   * address; 8-byte stores where it is 8-byte aligned); pass 2 reads it back (p_in 16-byte aligned)
+   * with blk_scale [B, Hkv, nb, G] */
   void* p_out;
   const void* p_in;
   const float* blk_scale;

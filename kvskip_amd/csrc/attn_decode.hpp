@@ -501,6 +501,9 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     const rsrc_t rs_sum = make_rsrc(STATS ? p.blk_sum + hq0 * p.nb : nullptr, STATS ? G * nb4 : 0);
     const rsrc_t rs_p = make_rsrc(STATS && p.p_out != nullptr ? p.p_out + hq0 * p.t_pad : nullptr,
                                   STATS && p.p_out != nullptr ? G * tp2 : 0);
+    // P goes out in 8-byte pieces where its base allows them (a caller's buffer need only be aligned to its
+    // fp16 elements; a head's rows are whole blocks)
+    const bool p_wide = (reinterpret_cast<uintptr_t>(p.p_out) & 7u) == 0;
     // offsets of a lane with nothing to store: past any range
     constexpr uint32_t OOB = 0x80000000u;
     const uint32_t v_stat = c16 < G && j4 == 0 ? c16 * nb4 : OOB, v_p = c16 < G ? c16 * tp2 + 8u * j4 : OOB;
@@ -539,11 +542,18 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         bstore_f32(st, rs_sum, vs, blk4);
         if (!LOAD_V || p.p_out != nullptr) {
           const uint32_t vp = blk >= 0 ? v_p : OOB;
+          if (p_wide) {
 #pragma unroll
-          for (int nt = 0; nt < 4; ++nt)
-            bstore_b64(u32x2{f2h(e[nt][0]) | static_cast<uint32_t>(f2h(e[nt][1])) << 16,
-                             f2h(e[nt][2]) | static_cast<uint32_t>(f2h(e[nt][3])) << 16},
-                       rs_p, vp + 32 * nt, 2 * t0);
+            for (int nt = 0; nt < 4; ++nt)
+              bstore_b64(u32x2{f2h(e[nt][0]) | static_cast<uint32_t>(f2h(e[nt][1])) << 16,
+                               f2h(e[nt][2]) | static_cast<uint32_t>(f2h(e[nt][3])) << 16},
+                         rs_p, vp + 32 * nt, 2 * t0);
+          } else {
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) bstore_u16(f2h(e[nt][i]), rs_p, vp + 32 * nt + 2 * i, 2 * t0);
+          }
         }
       }
       if constexpr (LOAD_V) {

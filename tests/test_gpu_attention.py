@@ -345,3 +345,40 @@ def test_masked_stats_gaps(gpu, num_splits):
     assert not torch.isnan(bmax).any() and not torch.isnan(bsum).any(), "a block was left unwritten"
     assert (bmax[~vis] == -math.inf).all() and (bsum[~vis] == 0).all()
     assert torch.equal(bmax[vis], dense[2].cpu()[vis]) and torch.equal(bsum[vis], dense[3].cpu()[vis])
+
+
+@pytest.mark.parametrize("D,G", [(128, 4), (64, 7)])
+@pytest.mark.parametrize("load_v", [False, True])
+@pytest.mark.parametrize("paged", [False, True])
+def test_p_buffer_alignment(gpu, D, G, load_v, paged):
+    """The C ABI takes a P buffer at any fp16 address: the same P as at a 16-byte aligned one, and nothing beside it."""
+    import ctypes
+
+    from kvskip_amd import _native
+
+    T, Hkv = 64 * 9 + 5, 2
+    nb = math.ceil(T / 64)
+    gq, gk, gv = to_gpu(*rand_qkv(2, Hkv * G, Hkv, T, D, seed=D + G)[:3])
+    pages = {}
+    if paged:
+        table, kp, vp = W.paged_pools([gk], [gv], 3)
+        gk, gv, pages = kp[0], vp[0], dict(block_table=table, T=T)
+    f32 = dict(dtype=torch.float32, device="cuda")
+    B, Hq = gq.shape[:2]
+    n = B * Hq * nb * 64
+    got = []
+    for shift in (0, 1, 2, 3, 4):
+        out = torch.empty(B, Hq, D, dtype=torch.bfloat16, device="cuda")
+        lse, bm, bs = torch.empty(B, Hq, **f32), torch.empty(B, Hq, nb, **f32), torch.empty(B, Hq, nb, **f32)
+        part = torch.empty(B * Hq * 2 * D, **f32), torch.empty(B * Hq * 2 * 2, **f32)
+        buf = torch.full((n + 16,), 7.0, dtype=torch.float16, device="cuda")
+        P = buf[shift:shift + n]
+        assert P.data_ptr() % 8 == 2 * shift % 8
+        a = E._decode_args(gq, gk, gv, D ** -0.5, None, None, 2, out if load_v else None, lse, bm, bs, None, P, *part, **pages)
+        _native.check(_native.lib().kvskip_decode(ctypes.byref(a), 1, int(load_v),
+                                                  torch.cuda.current_stream().cuda_stream))
+        assert (buf[:shift] == 7.0).all() and (buf[shift + n:] == 7.0).all()
+        got.append((P.clone(), lse, bm, bs))
+    for r in got[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(r, got[0]))
+    assert got[0][0].float().max().item() == 1.0 and bool((got[0][0].view(B, Hq, -1)[..., T:] == 0).all())
