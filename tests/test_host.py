@@ -8,6 +8,7 @@ import torch
 
 from kvskip_amd import _native, ext
 from kvskip_amd import kvskip as K
+from kvskip_amd import planner as P
 
 
 def _rule(bh, n_tiles, slots, max_splits, min_tiles):
@@ -43,6 +44,24 @@ def test_zeroed_state():
         assert t.is_contiguous() and not t.any()
         t.fill_(i + 1)
     assert all((t == i + 1).all() for i, t in enumerate(ts))
+
+
+def test_grown_state_keeps_no_old_storage():
+    """A planner's state grown to another capacity holds the memory of its tensors (each padded to 256 bytes) and none
+    of the replaced ones', with the values carried over."""
+    p = P.FusedPlanner(P.Policy(dense_heads=(1,)), count=False)
+    B, Hkv, G, D, cap = 3, 4, 4, 64, 900
+    p._alloc(torch.zeros(B, Hkv * G, D), torch.zeros(B, Hkv, 64, D), cap)
+    for i, x in enumerate(p.state.values()):
+        x.fill_(i + 1)
+    old = {x: t.clone() for x, t in p.state.items()}
+    p._grow(2 * cap)
+    held = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for t in p.state.values()}
+    need = sum((t.numel() * t.element_size() + 255) // 256 * 256 for t in p.state.values())
+    assert sum(held.values()) <= need
+    for x, t in p.state.items():
+        if x not in ("part", "idx"):                 # a workspace; rewritten by every step
+            assert torch.equal(t[:, :, :cap] if t.dim() > 2 else t, old[x]), x
 
 
 def test_refusals():
