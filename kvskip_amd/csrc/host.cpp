@@ -117,6 +117,7 @@ PyObject* list_of(std::initializer_list<at::Tensor> ts) {
 // Device guard and current stream of a launch; the launch itself runs without the interpreter lock.
 template <class F>
 void launch(const at::Device& dev, F&& f) {
+  TORCH_CHECK_VALUE(dev.is_cuda(), "Expected a cuda device, but got: ", dev.str());
   c10::DeviceGuard guard(dev);
   PyObject* i = PyLong_FromLong(dev.index());
   PyObject* s = i != nullptr ? PyObject_CallOneArg(raw_stream, i) : nullptr;

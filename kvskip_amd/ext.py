@@ -39,8 +39,10 @@ _host = _native.host      # the native argument checks, allocations and launches
 
 
 def _device_index(device) -> int:
-    i = torch.device(device).index
-    return torch.cuda.current_device() if i is None else i
+    d = torch.device(device)
+    if d.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {d}")
+    return torch.cuda.current_device() if d.index is None else d.index
 
 
 def _stream(dev: torch.device):

@@ -1,5 +1,6 @@
 """CPU checks of the native host module (csrc/host.cpp): the split rule count by count, zeroed state
 carved from one allocation, and refusals with the messages that the Python checks had."""
+import ctypes
 import math
 import random
 
@@ -77,4 +78,15 @@ def test_refusals():
                       (lambda: ext.plan(q, k, *[f] * 11, 0.1, 0.1, 1, 2, True), "q: CUDA bf16"),
                       (lambda: ext.decode_into(q, k, k, 0.1, {}), "q must be CUDA bf16")):
         with pytest.raises(RuntimeError, match=msg):
+            call()
+
+
+def test_launches_refuse_other_devices():
+    """A launch goes to the tensor's own CUDA device: host memory is refused before anything is launched."""
+    plan, upd, attn = _native.PlanArgs(), _native.UpdateArgs(), _native.AttnArgs()
+    host, q = _native.host(), torch.zeros(1, 32, 128)
+    for call in (lambda: ext.launch_update(upd, torch.device("cpu")), lambda: ext.plan_scores(plan, "cpu"),
+                 lambda: host.plan(ctypes.addressof(plan), q),
+                 lambda: host.merge_update(ctypes.addressof(attn), ctypes.addressof(upd), q)):
+        with pytest.raises(ValueError, match="Expected a cuda device, but got: cpu"):
             call()
