@@ -35,7 +35,10 @@ enum {
 
 /* Attention launch block: replaces kvskip::Params (kernels/kvskip.h:13-60).
  * q [B, Hq, D] bf16; k, v [B, Hkv, T, D] bf16 with arbitrary batch/head/token element
- * strides, D contiguous, all strides multiples of 8 elements, base 16-byte aligned. */
+ * strides, D contiguous, all strides multiples of 8 elements, base 16-byte aligned.
+ * The last bits of a sequence's results follow its length (or lists), num_splits, the index of its
+ * KV head and, with seq_lens or kvskip_plan_args.pass_budget, the batch's other lengths (they set
+ * the cut); not its slot in the batch, the strides, or whether the cache is paged. */
 typedef struct kvskip_attn_args {
   const void* q;
   const void* k;

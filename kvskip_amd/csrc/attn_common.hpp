@@ -298,19 +298,24 @@ __device__ int global_lookup(const AttnP& p, int it, int& b, int& h, int& chunk,
 // rotation below short).
 constexpr int LONG_BLOCKS = 24;
 
-// Item of step k of a wavefront with nw > 0 items: k rotated by the workgroup's place in the grid (b, h and
-// the split alone, so passes that cut alike add alike). Without it every workgroup starts at the same
-// offset of its own range, and where the ranges lie at multiples of the memory's channel interleave apart
-// all of them read the same few channels at a time: B 1 at 64k in a buffer of 66048 tokens 74.0 -> 46.3 us
-// per op, of 65536 48.7 -> 45.4, B 2 at 64k (66048) 104.8 -> 85.7, single-pass V-skip at 64k 37.8 -> 26.3;
-// other short ones within 1%. Long streams drift apart by themselves, and spread further they lose locality:
-// rotated by up to 4 of their items B 8 at 64k takes 318 us, B 32 at 64k 1221 and at 60k 1113 (none: 328,
-// 1225, 1109; by up to all of them 312, 1242, 1110). Where a head is one split the choice
-// depends on the stride: B 32 at 65536 1246 - 1269 us (none 1270 - 1302), at 48000 of 49152 945 - 951 (962 -
-// 976), at 65552 of 65568 1276 - 1301 (1233 - 1265).
-__device__ __forceinline__ int item_rotation(const AttnP& p, int b, int h, int split, int nw) {
+// Item of step k of a wavefront with nw > 0 items: k rotated by the workgroup's place among its sequence's (the
+// KV head and the split alone: a sequence adds its blocks in the same order in every batch slot and wherever its
+// rows lie, over pages too, and passes that cut alike add alike; decode_body adds a ragged batch's item counts).
+// Without it every workgroup starts at the same offset of its own range, and where the ranges lie at multiples of
+// the memory's channel interleave apart all of them read the same few channels at a time: B 1 at 64k in a buffer of
+// 66048 tokens 61 -> 44.2 us per op, B 2 107 -> 81.4, single-pass V-skip at 64k 40.8 -> 24.4, B 64 at 2048 85.7 ->
+// 79.3; other short ones within 2%.
+// Long streams drift apart by themselves, and spread further they lose locality: they rotate by up to 4 of their
+// items. B 8 at 64k 319.5 us (none: 325). Where a head is one split the ranges are a head stride apart and the gain
+// depends on it (B 32 unless given, tokens of the buffer, us, rotated / not): 36864 697 / 722, 40960 816 / 858,
+// 49152 965 / 1000, 65536 1268 / 1290, D 64 98304 940 / 1049; but 32784 617 / 607, 65568 1273 / 1262, 65792
+// 1293 / 1277, 69632 1442 / 1429, B 64 at 32768 1300 / 1267; elsewhere within 0.5%. Rotated where the stride asks
+// for it only, the sums' order would follow the buffer's shape, and pages would no longer give the contiguous
+// cache's bits. By up to 3: D 64 98304 961, 65568 1281, 65792 1282, B 64 1269, else the same; by 8: 32784 651, 65568
+// 1283, 49152 954, D 64 98304 919.
+__device__ __forceinline__ int item_rotation(const AttnP& p, int h, int split, int nw) {
   const int span = nw < LONG_BLOCKS ? nw : 4;
-  return nw > 0 ? __builtin_amdgcn_readfirstlane(((b * p.Hkv + h) * p.num_splits + split) % span) : 0;
+  return nw > 0 ? __builtin_amdgcn_readfirstlane((h * p.num_splits + split) % span) : 0;
 }
 __device__ __forceinline__ int rotated(int k, int rot, int nw) {
   const int i = min(k, nw - 1) + rot;

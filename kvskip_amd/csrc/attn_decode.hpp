@@ -457,7 +457,9 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
   if constexpr (PAGED)
     gather_pages(p, b, n, nbb, [&](int t) { return MASKED ? list(i0 + t) : i0 + t; }, sPg, MASKED ? sBk : nullptr);
   const int nw = n > wave ? (n - wave + NWAVE - 1) / NWAVE : 0;  // this wavefront's items
-  const int rot = item_rotation(p, b, h, split, nw);
+  // over a ragged batch the sequences (lists) start at places of their own by their lengths: 24 of up to 32000
+  // tokens, 20% listed, 55.0 -> 52.1 us, 16 of 7 heads dense 137.3 -> 134.8
+  const int rot = item_rotation(p, h, split + (RAG && p.B > 1 ? n_items : 0), nw);
   // paged: item of step k of this wavefront (LDS slot wave + NWAVE item): its block and page
   auto paged_item = [&](int k, int& blk, int& pg) {
     const int t = wave + NWAVE * rotated(k, rot, nw);

@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(NT, 2) vskip1_kernel(const AttnP p) {
     // keeps the block. Measured (op, us; B 8 at 32k nothing kept / 64k peaked): the P V by FMAs and K
     // requested after the vote 98.3 / 44.6; P V on MFMA 93.9 / 42.2; K requested after the scores 91.8 /
     // 42.2. V requested always (out of range where not kept) and used a step later: 113.0.
-    const int rot = item_rotation(p, b, h, split, nw);
+    const int rot = item_rotation(p, h, split, nw);
     auto slot_of = [&](int k) { return wave + NWAVE * rotated(k, rot, nw); };  // of step k: block i0 + slot
     int pg = nw > 0 ? page_at(slot_of(0)) : -1;
     if (nw > 0) load_k_block_mf<D>(kr, krs(i0 + slot_of(0), pg), koffm, p.k_st, (i0 + slot_of(0)) * BLK);

@@ -39,3 +39,35 @@ def test_streams(gpu, D, G, T, S):
     a = K.decode(gq, gk, gv, sc, num_splits=S)
     b = K.decode(gq, kp[0], vp[0], sc, num_splits=S, block_table=table, T=T)
     assert torch.equal(a["out"], b["out"]) and torch.equal(a["lse"], b["lse"])
+
+
+@pytest.mark.parametrize("D,G", [(128, 4), (64, 7)])
+@pytest.mark.parametrize("T,S", [(64 * 4 * 6, 1), (64 * 5 * 4 + 9, 2), (64 * 4 * 26, 1), (64 * 4 * 2 * 25 + 1, 2), (64 * 45, 3)])
+def test_batch_slots_alike(gpu, D, G, T, S):
+    """A sequence gives the same bits in every slot of a batch and in buffers of any capacity: short and long streams, one
+    and several splits, each pass that rotates its steps."""
+    B, Hkv = 5, 3
+    g = torch.Generator().manual_seed(T + G)
+    cap = (T + 2047) // 2048 * 2048
+    q = torch.randn(1, Hkv * G, D, generator=g).to(torch.bfloat16).cuda().expand(B, -1, -1).contiguous()
+    keep = W.random_block_list(1, Hkv, (T + 63) // 64, 0.6, seed=T).cuda().expand(B, -1, -1).contiguous()
+    lens = torch.full((B,), T, dtype=torch.int32, device="cuda")
+    plan = K.make_plan(keep)
+    rows = [torch.randn(1, Hkv, T, D, generator=g).to(torch.bfloat16).cuda() for _ in range(2)]
+    first = None
+    for tokens in (cap, cap + 64):
+        k, v = (torch.zeros(B, Hkv, tokens, D, dtype=torch.bfloat16, device="cuda")[:, :, :T].copy_(x) for x in rows)
+        table, kp, vp = W.paged_pools([k], [v], 3)
+        sc = D ** -0.5
+        runs = [K.decode(q, k, v, sc, out_f32=True, num_splits=S),
+                K.decode(q, k, v, sc, out_f32=True, num_splits=S, stats=True, plan=plan),
+                K.decode(q, kp[0], vp[0], sc, out_f32=True, num_splits=S, block_table=table, T=T),
+                K.decode(q, k, v, sc, out_f32=True, num_splits=max(S, 2) * B, seq_lens=lens),
+                K.decode(q, k, v, sc, stats=True, load_v=False, num_splits=S),
+                K.vskip_one_pass(q, k, v, sc, tau=1e-4, out_f32=True, num_splits=S, sync=False)]
+        for r in runs:
+            for x in ("out_f32", "lse"):
+                if x in r:
+                    assert all(torch.equal(r[x][b], r[x][0]) for b in range(1, B)), x
+        first = first or runs
+        assert all(torch.equal(r[x], f[x]) for r, f in zip(runs, first) for x in ("out_f32", "lse") if x in r)
