@@ -43,6 +43,37 @@ def test_key_sums(gpu, G, D):
         assert (sums[b, :, m:] == 7.0).all()
 
 
+@pytest.mark.parametrize("G,D", [(4, 128), (8, 64), (8, 128)])
+def test_key_sums_of_long_streams(gpu, G, D):
+    """The same where a wavefront streams 24 blocks and more (its steps then rotate by up to 4 alone, and a pass without
+    the sums takes K another way): one and several chunks a sequence, ragged last blocks."""
+    lens = [64 * 430 + 17, 64, 64 * 210, 64 * 100 + 1]
+    B, Hkv, T, S = len(lens), 2, max(lens), 3
+    g = torch.Generator().manual_seed(G * D)
+    q = torch.randn(B, Hkv * G, D, generator=g).to(torch.bfloat16).cuda()
+    k, v = (torch.randn(B, Hkv, T, D, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    nb, f32 = (T + 63) // 64, dict(dtype=torch.float32, device="cuda")
+    bufs = dict(out=torch.empty(B, Hkv * G, D, dtype=torch.bfloat16, device="cuda"), lse=torch.empty(B, Hkv * G, **f32),
+                blk_max=torch.empty(B * Hkv * G * nb, **f32), blk_sum=torch.empty(B * Hkv * G * nb, **f32),
+                part_acc=torch.empty(B * Hkv * G * S * D, **f32), part_ml=torch.empty(B * Hkv * G * S * 2, **f32))
+    ref = {x: y.clone() for x, y in bufs.items()}
+    sums = torch.full((B, Hkv, nb + 2, D), 7.0, **f32)
+    E.decode_into(q, k, v, D ** -0.5, bufs, stats=True, num_splits=S, seq_lens=sl, key_sums=sums)
+    E.decode_into(q, k, v, D ** -0.5, ref, stats=True, num_splits=S, seq_lens=sl)
+    for x in ("out", "lse"):
+        assert torch.equal(bufs[x], ref[x]), x
+    for b, n in enumerate(lens):
+        m = (n + 63) // 64
+        pad = torch.zeros(Hkv, m * 64, D, dtype=torch.float64)
+        pad[:, :n] = k[b, :, :n].cpu().double()
+        assert (sums[b, :, :m].cpu().double() - pad.view(Hkv, m, 64, D).sum(2)).abs().max().item() <= 1e-5 * 8
+        assert (sums[b, :, m:] == 7.0).all()
+        for x in ("blk_max", "blk_sum"):
+            y, z = (t[x].view(B, Hkv * G, nb)[b, :, :m] for t in (bufs, ref))
+            assert torch.equal(y, z), x
+
+
 @pytest.mark.parametrize("ragged", [False, True])
 def test_first_step(gpu, monkeypatch, ragged):
     """A batch's planner from a first step with the sums in its pass, against one with block_sums: the same decisions,

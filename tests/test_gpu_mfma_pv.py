@@ -5,6 +5,7 @@ import torch
 
 from kvskip_amd import ext as E
 from kvskip_amd import kvskip as K
+from kvskip_amd import planner as P
 from kvskip_amd import workloads as W
 from oracle import attention as O
 
@@ -68,9 +69,11 @@ def test_infinite_values_of_light_tokens(gpu, G, D, score):
     outs += [K.decode(q, k, v, 1.0, out_f32=True, num_splits=2, seq_lens=lens)["out_f32"],
              K.decode(q, kp[0], vp[0], 1.0, out_f32=True, num_splits=2, block_table=table, T=T)["out_f32"],
              K.vskip_one_pass(q, k, v, 1.0, local=nb, out_f32=True, num_splits=1)["out_f32"],
-             K.vskip_one_pass(q, kp[0], vp[0], 1.0, local=nb, out_f32=True, num_splits=2, block_table=table, T=T)["out_f32"]]
+             K.vskip_one_pass(q, kp[0], vp[0], 1.0, local=nb, out_f32=True, num_splits=2, block_table=table, T=T)["out_f32"],
+             P.FusedPlanner(P.Policy(), count=False).first(q, k, v, 1.0),
+             P.FusedPlanner(P.Policy(), count=False).first(q, kp[0], vp[0], 1.0, block_table=table, T=T)]
     for o in outs:
-        o = o.cpu()
+        o = o.float().cpu()
         want = torch.zeros_like(o, dtype=torch.bool)
         want[0, :G, 3] = want[0, G:, D - 1] = True
         assert not o.isnan().any() and torch.equal(o.isinf(), want)
@@ -86,18 +89,18 @@ def test_pv_weights_of_any_sign(gpu, G, D, S):
     g = torch.Generator().manual_seed(10 * G + S)
     Hkv, T = 2, 300
     nb = (T + 63) // 64
-    P = torch.rand(1, Hkv * G, nb * 64, generator=g).half()
-    P[torch.rand(P.shape, generator=g) < 0.5] = 0.0
-    P[:, :, T:] = 0.0
-    P[0, :, 5] = 1.0
+    p = torch.rand(1, Hkv * G, nb * 64, generator=g).half()
+    p[torch.rand(p.shape, generator=g) < 0.5] = 0.0
+    p[:, :, T:] = 0.0
+    p[0, :, 5] = 1.0
     v = torch.randn(1, Hkv, T, D, generator=g).to(torch.bfloat16)
     sc = torch.randn(1, Hkv, nb, G, generator=g)
     sc[0, :, 0] = 2.0 ** -112
     sc[0, :, 2] = -sc[0, :, 2].abs()
     every = K.make_plan(torch.ones(1, Hkv, nb, dtype=torch.bool, device="cuda"))
-    args = (P.cuda(), sc.cuda(), every.block_idx, every.block_cnt)
+    args = (p.cuda(), sc.cuda(), every.block_idx, every.block_cnt)
     out = E.pv(args[0], v.cuda(), *args[1:], S, True)[1].cpu().double()
-    w = (P.double().view(Hkv, G, nb, 64) * sc[0].double().transpose(1, 2)[..., None]).reshape(Hkv, G, -1)[..., :T]
+    w = (p.double().view(Hkv, G, nb, 64) * sc[0].double().transpose(1, 2)[..., None]).reshape(Hkv, G, -1)[..., :T]
     ref, mag = torch.matmul(w, v[0].double()).view(1, -1, D), torch.matmul(w.abs(), v[0].double().abs()).view(1, -1, D)
     assert not out.isnan().any()
     assert float((out - ref).norm() / mag.norm()) <= F32_REL
