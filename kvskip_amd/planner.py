@@ -179,17 +179,14 @@ class FusedPlanner:
         f32 = dict(dtype=torch.float32, device=dev)
         self.NBC = NBC
         BH, heads, qheads = ("i4", (B * Hkv,)), (B, Hkv), (B, Hq)
-        # two allocations, one fill each: what _grow replaces (its memory is then given back), and the rest
-        blocks = dict(cs_ref=("f4", (*qheads, NBC)), cs_now=("f4", (*qheads, NBC)), keep=("u1", (*heads, NBC)),
-                      block_idx=("i4", (*heads, NBC)), idx=("u1", (B, NBC)))
-        rest = dict(lse_att=("f4", qheads), age=("i4", heads), flags=("i4", (Hkv,)), trig=("u1", heads),
-                    block_cnt=("i4", heads), calib=("f4", heads), est=("f4", heads), aix=("u1", heads),
+        zero = dict(cs_ref=("f4", (*qheads, NBC)), cs_now=("f4", (*qheads, NBC)), keep=("u1", (*heads, NBC)),
+                    lse_att=("f4", qheads), age=("i4", heads), flags=("i4", (Hkv,)), trig=("u1", heads),
+                    block_idx=("i4", (*heads, NBC)), block_cnt=("i4", heads), calib=("f4", heads), est=("f4", heads),
+                    aix=("u1", heads), idx=("u1", (B, NBC)),
                     tlen=("i4", (B,)),              # this step's lengths (ragged)
                     lens=("i4", (B,)),              # all T, for batch_balance
                     ticket=BH)                      # one-launch plan (self-resetting)
-        self.state = {}
-        for zero in (blocks, rest):
-            self.state.update(zip(zero, E._host().zeroed(tuple(zero.values()), q)))
+        self.state = dict(zip(zero, E._host().zeroed(tuple(zero.values()), q)))      # one allocation, one fill
         self.state.update(
             csum=torch.empty(B, Hkv, NBC, D, **f32),            # block_sums writes every block
             lse_ref=torch.full((B, Hq, NBC), -math.inf, **f32),
@@ -211,6 +208,11 @@ class FusedPlanner:
         B, Hq = self.state["lse_att"].shape
         Hkv = self.state["keep"].shape[1]
         self.state["part"] = torch.empty(E.plan_part_floats(B, Hq, Hkv, NBC), dtype=torch.float32, device=idx.device)
+        # the tensors that keep their sizes leave _alloc's one allocation too, so that its memory is given back (two
+        # allocations there instead cost the first step 15 us a layer)
+        for key, x in self.state.items():
+            if key not in fills and key not in ("idx", "part"):
+                self.state[key] = x.clone()
         self.NBC = NBC
 
     def _attend(self, q, k, v, scale, nb, seq_lens=None, key_sums=None):
