@@ -267,12 +267,11 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
   // 16 nt + 4 (lane / 16) .. + 3 of a block (mf_tok)
   const int hd = (lane & 15) % gpad<G>(), g = min(hd, G - 1);
   const bool used = hd < G && part_used<G>(lane);
-  // Items i0 + wave + 4k of this wavefront through a ring of R buffers: V, P and the scale of the
-  // next R - 1 items are in flight while item k is accumulated (R = 2: a third buffer measured
-  // slower, 21.7 vs 20 us at config 2's shape); list entries are loaded two items before their blocks (waiting for an entry
-  // never waits for block loads issued after it). Every step issues the same loads; past the last
-  // item they read nothing from memory (below) and nothing is accumulated.
-  constexpr int R = 2;
+  // Items i0 + wave + 4k of this wavefront through two buffers: V, P and the scale of the next item are in
+  // flight while item k is accumulated (a third buffer measured slower, 21.7 vs 20 us at config 2's shape);
+  // list entries are loaded two items before their blocks (waiting for an entry never waits for block loads
+  // issued after it). Every step issues the same loads; past the last item they read nothing from memory
+  // (below) and nothing is accumulated.
   const int nw = n > wave ? (n - wave + NWAVE - 1) / NWAVE : 0;
   auto entry_of = [&](int k) -> int { return list_at(i0 + wave + NWAVE * min(k, nw - 1)); };
   auto block_of = [&](int e) -> int {
@@ -312,7 +311,7 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
   };
   if constexpr (PAGED) gather_pages(p, b, n, p.nb, [&](int t) { return list_at(i0 + t); }, sPg, sBk);
   if (PAGED && nw > 0) {
-    // the same ring over the LDS copy of this split's entries and their pages
+    // the same two buffers over the LDS copy of this split's entries and their pages
     Item I0, I1;
     auto item = [&](int k, int& blk, int& pgv) {
       if (k < nw) {
@@ -339,15 +338,14 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
       step(I0, b0, g0, I1, b1, k + 1);
     }
   } else if (nw > 0) {
-    Item I0, I1, I2;
-    int ea = entry_of(R - 1), eb = entry_of(R);
-    int b0 = block_of(entry_of(0)), b1 = R > 2 && nw > 1 ? block_of(entry_of(1)) : PAST, b2 = PAST;
+    Item I0, I1;
+    int ea = entry_of(1), eb = entry_of(2);
+    int b0 = block_of(entry_of(0)), b1 = PAST;
     load(I0, b0);
-    if constexpr (R > 2) load(I1, b1);
-    // step k: the blocks of item k + R - 1 into `ld` (its block into bld), then item k from `ac`
+    // step k: item k + 1 into `ld` (its block into bld), then item k from `ac`
     auto step = [&](Item& ld, int& bld, const Item& ac, int bac, int k) {
-      const int ec = entry_of(k + R + 1);
-      bld = k + R - 1 < nw ? block_of(ea) : PAST;
+      const int ec = entry_of(k + 3);
+      bld = k + 1 < nw ? block_of(ea) : PAST;
       ea = eb;
       eb = ec;
       load(ld, bld);
@@ -355,17 +353,9 @@ __device__ __forceinline__ void pv_body(const AttnP& p, int split, int h, int b,
       if (k < nw) accumulate(ac, bac);
       __builtin_amdgcn_sched_barrier(0);
     };
-    if constexpr (R > 2) {
-      for (int k = 0; k < nw; k += 3) {
-        step(I2, b2, I0, b0, k);
-        step(I0, b0, I1, b1, k + 1);
-        step(I1, b1, I2, b2, k + 2);
-      }
-    } else {
-      for (int k = 0; k < nw; k += 2) {
-        step(I1, b1, I0, b0, k);
-        step(I0, b0, I1, b1, k + 1);
-      }
+    for (int k = 0; k < nw; k += 2) {
+      step(I1, b1, I0, b0, k);
+      step(I0, b0, I1, b1, k + 1);
     }
   }
   finish_mf<D, G, true>(p, 0.f, 1.f, acc, b, h, split, sL, true);

@@ -6,7 +6,8 @@
 // Python): a decode of 200 tokens, whose kernel takes 6 us, 20.1 -> 7.9; B 1 at 32k 67.9 -> 25.7 (the
 // kernels' time); single-pass V-skip at 64k 87.6 -> 41.5; four layers x 12 planner steps at 32k
 // 6800 -> 1830.
-// Nothing is kept from one call to the next but the entry points' addresses (bind).
+// Nothing is kept from one call to the next but what bind() was given: the entry points' addresses and
+// torch's function of the current stream.
 #include <Python.h>
 
 #include <ATen/ops/empty.h>

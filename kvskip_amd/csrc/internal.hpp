@@ -94,11 +94,11 @@ bool attn_supported(int D, int G);
 hipError_t launch_decode(const AttnP& p, int D, int G, bool masked, bool stats, bool load_v, int phase,
                          hipStream_t s);
 // launch_decode over a paged cache (p.block_table set; the MFMA engine), same phases.
-// The dense ragged pass with statistics and key sums ([B, Hkv, cap, D], kvskip_attn_args.key_sums): phase 1
-// its split pass, 3 with the merge.
-hipError_t launch_decode_sums(const AttnP& p, int D, int G, float* sums, int cap, int phase, hipStream_t s);
 hipError_t launch_decode_paged(const AttnP& p, int D, int G, bool masked, bool stats, bool load_v, int phase,
                                hipStream_t s);
+// The dense ragged pass with statistics and key sums ([B, Hkv, cap, D], kvskip_attn_args.key_sums; the MFMA
+// engine, as every ragged pass): phase 1 its split pass, 3 with the merge.
+hipError_t launch_decode_sums(const AttnP& p, int D, int G, float* sums, int cap, int phase, hipStream_t s);
 hipError_t launch_vskip1(const AttnP& p, int D, int G, hipStream_t s);
 hipError_t launch_pv(const AttnP& p, int D, int G, hipStream_t s);
 // Two-pass V-skip pass 2 with the selection of sel in its prologue (then its split merge).

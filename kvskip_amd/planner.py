@@ -32,9 +32,11 @@ BALANCE_MAX_LISTS = 16           # (b, KV head) lists a balanced planned pass de
 RAGGED_DECIDE_MAX_B = 16         # sequences of a ragged batch whose lists a planned pass decides per KV head
 GLOBAL_PARTITION_MAX_LISTS = 512  # B * Hkv bound of kvskip_attn_args.list_partition = 1
 GLOBAL_PARTITION_MAX_B = 64        # sequences up to which the planner cuts all heads' lists together
-# Blocks of K (B * Hkv * nb; 256 MiB of 128-dim keys) from which on a batch's first step sums the keys in its dense
-# pass instead of a pass of their own: below, K is still in the cache for the second reading and the update rides
-# on the next layer's pass instead of beside the merge
+# Blocks of K (B * Hkv * nb) from which on a batch's first step sums the keys in its dense pass instead of a pass
+# of their own. A layer's first step, us, apart / in the pass: 8 x 16400 tokens of 8 KV heads (16448 blocks) 162.5 /
+# 125.3, of 64 dims 92.6 / 77.9, ragged 88.6 / 69.9. What the pass of their own has for it, a second reading of K from
+# the cache and an update that rides on the next layer's pass, does not outweigh that at smaller sizes either (8 x 8k,
+# 8000 blocks, 91.2 / 71.9, of 64 dims 59.1 / 49.9), so the line could lie lower
 SUMS_IN_PASS_BLOCKS = 16384
 POST_MAX_SLOTS = 64              # first-pass partial slots the refresh mode's decision reads (lse_slots)
 KINDS = {"logit": 0, "add": 1, "peak": 2}
