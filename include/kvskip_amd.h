@@ -87,8 +87,8 @@ typedef struct kvskip_attn_args {
    * nb = ceil(T / 64) sizes the statistics). The split pass then partitions each KV head's work
    * over the whole batch: chunks of C = ceil(sum_b items_b / num_splits) blocks (or list entries),
    * so every workgroup gets at most C whatever the lengths; needs num_splits >= 2, B <= 256, and
-   * part_acc / part_ml of [B, Hq, num_splits, ...]. Always the MFMA engine, as over a paged cache
-   * (KVSKIP_AMD_QK=valu does not apply). */
+   * part_acc / part_ml of [B, Hq, num_splits, ...]. Always the MFMA engine, whatever
+   * KVSKIP_AMD_QK says. */
   const int32_t* seq_lens;
 
   /* Paged cache (not in the reference; every pass that reads K or V: kvskip_decode and its split
