@@ -504,8 +504,8 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     const rsrc_t rs_p = make_rsrc(STATS && p.p_out != nullptr ? p.p_out + hq0 * p.t_pad : nullptr,
                                   STATS && p.p_out != nullptr ? G * tp2 : 0);
     // P goes out in 8-byte pieces where its base allows them (a caller's buffer need only be aligned to its
-    // fp16 elements; a head's rows are whole blocks)
-    const bool p_wide = (reinterpret_cast<uintptr_t>(p.p_out) & 7u) == 0;
+    // fp16 elements; a head's rows are whole blocks; a ragged batch has no P)
+    const bool p_wide = RAG || (reinterpret_cast<uintptr_t>(p.p_out) & 7u) == 0;
     // offsets of a lane with nothing to store: past any range
     constexpr uint32_t OOB = 0x80000000u;
     const uint32_t v_stat = c16 < G && j4 == 0 ? c16 * nb4 : OOB, v_p = c16 < G ? c16 * tp2 + 8u * j4 : OOB;
@@ -517,8 +517,9 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
     // block blk's scores (tokens >= lim masked: lim = Tb, or 0 for an empty block), statistics and P;
     // pf: its weights, alpha: the accumulators' rescale (this lane's head's). next_k: the K loads of the
     // block after it, into the registers its scores have just left. (Issued after the softmax: B 8 at 32k
-    // 157.9 against 155.0 us per op; after P V: 159.7.)
-    auto process = [&](auto staged, int blk, int lim, const u32x4 (&kr)[4][KS], PFrag<G>& pf, float& alpha,
+    // 157.9 against 155.0 us per op; after P V: 159.7.) wide: p_wide, known at compile time in the passes
+    // over K alone.
+    auto process = [&](auto staged, auto wide, int blk, int lim, const u32x4 (&kr)[4][KS], PFrag<G>& pf, float& alpha,
                        auto&& next_k) {
       const int t0 = blk >= 0 ? blk * BLK : 0;
       float s[4][4], e[4][4];
@@ -544,7 +545,7 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
         bstore_f32(st, rs_sum, vs, blk4);
         if (!LOAD_V || p.p_out != nullptr) {
           const uint32_t vp = blk >= 0 ? v_p : OOB;
-          if (p_wide) {
+          if (wide) {
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt)
               bstore_b64(u32x2{f2h(e[nt][0]) | static_cast<uint32_t>(f2h(e[nt][1])) << 16,
@@ -581,58 +582,69 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
       bstore16_f32(ks[0], ks[1], ks[2], ks[3], rs_ks, off, so);
       bstore16_f32(ks[4], ks[5], ks[6], ks[7], rs_ks, off + 16, so);
     };
-    if (nw > 0 && !LOAD_V && PAGED) {
-      // K only over a paged cache: two blocks in flight as below, each through its page's resource
-      u32x4 ka[4][KS], kb[4][KS];
-      int b0, g0, b1 = -1, g1 = -1;
-      paged_item(0, b0, g0);
-      load_k_block_mf<D>(ka, block_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, h, b0, g0, Tb, D), koffm, p.k_st,
-                         max(b0, 0) * BLK);
-      auto step = [&](u32x4 (&ld)[4][KS], int& bld, int& gld, const u32x4 (&ac)[4][KS], int bac, int gac, int k) {
-        if (k + 1 < nw) {
-          paged_item(k + 1, bld, gld);
-        } else {
-          bld = -1;
-          gld = -1;
+    // The passes over K alone, the width of the P stores a parameter of the whole loop (a branch on it around
+    // the stores made the waits for K cover up to four of the next block's loads: two-pass V-skip, 4 x 40k, its
+    // first pass 58.3 -> 58.9 us).
+    auto k_only = [&](auto wide) {
+      if constexpr (PAGED) {
+        // K only over a paged cache: two blocks in flight as below, each through its page's resource
+        u32x4 ka[4][KS], kb[4][KS];
+        int b0, g0, b1 = -1, g1 = -1;
+        paged_item(0, b0, g0);
+        load_k_block_mf<D>(ka, block_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, h, b0, g0, Tb, D), koffm, p.k_st,
+                           max(b0, 0) * BLK);
+        auto step = [&](u32x4 (&ld)[4][KS], int& bld, int& gld, const u32x4 (&ac)[4][KS], int bac, int gac, int k) {
+          if (k + 1 < nw) {
+            paged_item(k + 1, bld, gld);
+          } else {
+            bld = -1;
+            gld = -1;
+          }
+          load_k_block_mf<D>(ld, block_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, h, bld, gld, Tb, D), koffm, p.k_st,
+                             max(bld, 0) * BLK);
+          __builtin_amdgcn_sched_barrier(0);
+          PFrag<G> pf;
+          float alpha;
+          process(std::true_type{}, wide, bac, (bac >= 0 && gac >= 0) ? Tb : 0, ac, pf, alpha, [] {});
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int k = 0; k + 1 < nw; k += 2) {
+          step(kb, b1, g1, ka, b0, g0, k);
+          step(ka, b0, g0, kb, b1, g1, k + 1);
         }
-        load_k_block_mf<D>(ld, block_rsrc(p.k, p.k_sb, p.k_sh, p.k_st, h, bld, gld, Tb, D), koffm, p.k_st,
-                           max(bld, 0) * BLK);
-        __builtin_amdgcn_sched_barrier(0);
-        PFrag<G> pf;
-        float alpha;
-        process(std::true_type{}, bac, (bac >= 0 && gac >= 0) ? Tb : 0, ac, pf, alpha, [] {});
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      for (int k = 0; k + 1 < nw; k += 2) {
-        step(kb, b1, g1, ka, b0, g0, k);
-        step(ka, b0, g0, kb, b1, g1, k + 1);
+        if (nw % 2 != 0) step(kb, b1, g1, ka, b0, g0, nw - 1);
+      } else {
+        // K only: two blocks in flight while one is scored (the V registers are free). Step k loads
+        // item k + 1 and scores item k; past the last item the load reads beyond the head's buffer
+        // range (zeros, no memory access), so every step issues the same loads.
+        u32x4 ka[4][KS], kb[4][KS];
+        int ea = entry_of(1), eb = entry_of(2);
+        int b0 = block_of(entry_of(0), 0), b1 = -1;
+        load_k_block_mf<D>(ka, rk, koffm, p.k_st, max(b0, 0) * BLK);
+        auto step = [&](u32x4 (&ld)[4][KS], int& bld, const u32x4 (&ac)[4][KS], int bac, int k) {
+          const int ec = entry_of(k + 3);
+          bld = block_of(ea, min(k + 1, nw - 1));
+          ea = eb;
+          eb = ec;
+          load_k_block_mf<D>(ld, rk, koffm, p.k_st, (k + 1 < nw ? max(bld, 0) : nbb) * BLK);
+          __builtin_amdgcn_sched_barrier(0);
+          PFrag<G> pf;
+          float alpha;
+          process(std::true_type{}, wide, bac, bac >= 0 ? Tb : 0, ac, pf, alpha, [] {});
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int k = 0; k + 1 < nw; k += 2) {
+          step(kb, b1, ka, b0, k);
+          step(ka, b0, kb, b1, k + 1);
+        }
+        if (nw % 2 != 0) step(kb, b1, ka, b0, nw - 1);
       }
-      if (nw % 2 != 0) step(kb, b1, g1, ka, b0, g0, nw - 1);
-    } else if (nw > 0 && !LOAD_V) {
-      // K only: two blocks in flight while one is scored (the V registers are free). Step k loads
-      // item k + 1 and scores item k; past the last item the load reads beyond the head's buffer
-      // range (zeros, no memory access), so every step issues the same loads.
-      u32x4 ka[4][KS], kb[4][KS];
-      int ea = entry_of(1), eb = entry_of(2);
-      int b0 = block_of(entry_of(0), 0), b1 = -1;
-      load_k_block_mf<D>(ka, rk, koffm, p.k_st, max(b0, 0) * BLK);
-      auto step = [&](u32x4 (&ld)[4][KS], int& bld, const u32x4 (&ac)[4][KS], int bac, int k) {
-        const int ec = entry_of(k + 3);
-        bld = block_of(ea, min(k + 1, nw - 1));
-        ea = eb;
-        eb = ec;
-        load_k_block_mf<D>(ld, rk, koffm, p.k_st, (k + 1 < nw ? max(bld, 0) : nbb) * BLK);
-        __builtin_amdgcn_sched_barrier(0);
-        PFrag<G> pf;
-        float alpha;
-        process(std::true_type{}, bac, bac >= 0 ? Tb : 0, ac, pf, alpha, [] {});
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      for (int k = 0; k + 1 < nw; k += 2) {
-        step(kb, b1, ka, b0, k);
-        step(ka, b0, kb, b1, k + 1);
-      }
-      if (nw % 2 != 0) step(kb, b1, ka, b0, nw - 1);
+    };
+    if constexpr (!LOAD_V) {
+      if (nw > 0 && p_wide)
+        k_only(std::true_type{});
+      else if (nw > 0)
+        k_only(std::false_type{});
     } else if (nw > 0) {
       auto stream = [&](auto staged) {
         constexpr bool ST = decltype(staged)::value;
@@ -659,7 +671,7 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
             const rsrc_t rv_n = page_rsrc(p.v, p.v_sb, p.v_sh, p.v_st, blk_n, pg_n);
             PFrag<G> pf;
             float alpha;
-            process(staged, blk, lim_of(blk, pg), kr, pf, alpha,
+            process(staged, p_wide, blk, lim_of(blk, pg), kr, pf, alpha,
                     [&] { load_k_block_mf<D, ST>(kr, rk_n, koff, p.k_st, max(blk_n, 0) * BLK); });
             accumulate(vr, pf, alpha);
             __builtin_amdgcn_sched_barrier(0);
@@ -683,7 +695,7 @@ __device__ __forceinline__ void decode_body(const AttnP& p, int bid, const kvski
             e_n = e_nn;
             PFrag<G> pf;
             float alpha;
-            process(staged, blk, blk >= 0 ? Tb : 0, kr, pf, alpha,
+            process(staged, p_wide, blk, blk >= 0 ? Tb : 0, kr, pf, alpha,
                     [&] {
                       if constexpr (SUMS) key_sums(blk, kr);
                       load_k_block_mf<D, ST>(kr, rk, koff, p.k_st, t_n);
