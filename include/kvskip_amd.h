@@ -126,7 +126,8 @@ typedef struct kvskip_attn_args {
  * statistics (stats), stats-only reading K alone (load_v = 0, needs stats) and fp16 P (p_out,
  * needs stats). num_splits (1..256) > 1 adds the log-sum-exp merge of the partials.
  * Replaces kvskip::launch_decode (kernels/kvskip.h:113-114, kernels/kvskip_kernel.cu:761-769),
- * reached from kvskip_ext.decode (kernels/kvskip_ext.cpp:25-101). Any G = Hq / Hkv in 1..8. */
+ * reached from kvskip_ext.decode (kernels/kvskip_ext.cpp:25-101). D in {64, 128}, G = Hq / Hkv in
+ * {1, 2, 4, 7, 8}; others are refused. */
 int kvskip_decode(const kvskip_attn_args* a, int stats, int load_v, void* stream);
 
 /* kvskip_decode as its two launches (num_splits >= 2; same arguments, called in this order on
@@ -167,7 +168,7 @@ int kvskip_read(const void* x, int64_t bytes, uint32_t* out, int32_t blocks, voi
 
 /* Refresh planner, before the attention pass. Replaces kvskip::PlanParams + launch_plan
  * (kernels/kvskip.h:63-89,115, kernels/kvskip_planner.cu:75-227,309-312), reached from
- * kvskip_ext.plan (kernels/kvskip_ext.cpp:205-267). Any D in {64, 128}, G in 1..8. */
+ * kvskip_ext.plan (kernels/kvskip_ext.cpp:205-267). D in {64, 128}, G in {1, 2, 4, 7, 8}. */
 typedef struct kvskip_plan_args {
   const void* q;               /* [B, Hq, D] bf16 */
   int64_t q_sb, q_sh;
